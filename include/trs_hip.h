@@ -239,7 +239,14 @@ int trs_accumulate_f32(float *dst, const float *src, size_t n);
 
 /* ---- matmul (Tensor::matmul, src/tensor.rs:2453-2533, 3872-3994) */
 
-/* C = A @ B in fp32 on CDNA4 FP32 MFMA.  Rank 2 ([M,K] @ [K,N]) or rank 3
+/* C = A @ B in fp32: fp32 operands, fp32 accumulation.  The tiled products
+ * run on the bf16 matrix cores with every float as the exact sum of three
+ * bf16 pieces and the six products of pieces of weight 2^-16 and above, the
+ * three left out being below 2^-24 of |a||b|; measured against 64 bits, the
+ * result is closer than fp32 MFMA's.  A tile that holds an infinity, a NaN, a
+ * nonzero value below 2^-110 with low bits set, or a sum that overflows is
+ * computed on fp32 MFMA instead.  Outputs with a side of at most 32 use fp32
+ * arithmetic throughout.  Rank 2 ([M,K] @ [K,N]) or rank 3
  * ([b,M,K] @ [b,K,N], the batch the reference spells as rank-2 calls).
  * Operands may be transposed views (unit stride in either matrix dim,
  * e.g. `.mT`).  An operand with no unit stride is first copied into a
@@ -249,8 +256,8 @@ int trs_accumulate_f32(float *dst, const float *src, size_t n);
  * must be contiguous.
  * Tolerance versus the reference's sequential order: |dC| <= 1e-5*sqrt(K) *
  * (|A||B|) elementwise.  A single matrix whose tiles would leave CUs idle
- * may split K into S slices summed in slice order: a 16-byte-aligned one
- * with M and N multiples of 256, fewer 256x256 tiles than CUs and a long K
+ * may split K into S slices summed in slice order: one
+ * with fewer 256x256 tiles than CUs, at least 90% covered, and a long K
  * (S <= 8, when S slices fill at least half the CUs or give at least as
  * many blocks as the unsplit tile), else one whose 128x128 or 64x128 tile
  * gives at most one block per CU (S <= 16, slices of at least 128 k).  The

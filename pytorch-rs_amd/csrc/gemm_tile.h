@@ -1,0 +1,517 @@
+// gemm_tile.h -- the tile body of the fp32 matmul: fp32 products on the bf16
+// matrix cores, three bf16 pieces per value.
+//
+// A float's 24 significant bits are the exact sum of three bf16 values:
+// h = rn(x), m = rn(x - h), l = x - h - m (bf16 has 8 significant bits and
+// float's exponent range, so nothing is scaled).  Of the nine products of
+// two such sums the six of weight 2^-16 and above are computed, each exact in
+// the matrix cores, and added into one fp32 accumulator, the small ones
+// first; the three left out are below 2^-24 of |x||y| together.  bf16 MFMA
+// runs 16 times the rate of fp32 MFMA, so six products cost 3/8 of the fp32
+// instruction's time.  Rounding to nearest matters: with truncated pieces
+// every small product has the sign of the whole one, and the accumulator's
+// alignment loses them in one direction (K = 4096 on positive data: 9.5e-6).
+//
+// Error against 64 bits (2-norm, relative; development probe, fp32 MFMA on
+// the same inputs in brackets): N(0,1) K = 16 3.3e-8 (7.4e-8), K = 256
+// 2.4e-7 (2.9e-7), K = 4096 1.01e-6 (1.15e-6); |N(0,1)| K = 4096 6.2e-7
+// (9.9e-7).
+//
+// Where the split does not hold -- a value whose lowest bits fall below
+// bf16's smallest subnormal (|x| < 2^-110 with low bits set), an infinity, a
+// NaN, a sum that overflows on the way -- the tile is computed again on fp32
+// MFMA (fp32_slots): the split notes lost bits as it goes, and everything
+// else leaves a non-finite accumulator.
+//
+// What bounds it: the card's power.  At 4096^3 a tile of zeros runs 416 us
+// (1,980 TFLOP/s of bf16), random values 570 us (1,445) at a lower clock; the
+// MFMAs alone on random values 466 us, with their LDS reads 490, with the
+// global loads 540.  The fp32 MFMA kernel this replaced took 945 us.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+namespace trs {
+
+typedef float gt_f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float gt_f2 __attribute__((ext_vector_type(2)));
+typedef float gt_f16 __attribute__((ext_vector_type(16)));
+typedef uint32_t gt_u4 __attribute__((ext_vector_type(4)));
+typedef const float __attribute__((address_space(1))) *gt_global;
+typedef const char __attribute__((address_space(1))) *gt_global_bytes;
+typedef __bf16 gt_bf2 __attribute__((ext_vector_type(2)));
+typedef __bf16 gt_bf8 __attribute__((ext_vector_type(8)));
+
+struct GemmArgs {
+    const float *a;
+    const float *b;
+    float *c;
+    int64_t M, N, K;
+    int64_t lda;  // stride of A's non-unit dim (rows if k-contiguous, k if not)
+    int64_t ldb;  // stride of B's non-unit dim (k if plain, columns if k-contiguous)
+    int64_t ldc;
+    int64_t bsa, bsb, bsc;  // batch strides (elements)
+    int64_t batch;
+    // Split K (batches are K slices of depth K): the full depth, so the last
+    // slice stops at ktotal; 0 when every batch has depth K.
+    int64_t ktotal;
+    int32_t tiles_m, tiles_n;
+    int32_t xcd_remap;
+    // Stream-K: blocks, slices per tile, (tile, slice) units, the k per
+    // slice, and the workspace of two partial tiles per block.
+    int64_t sk_blocks, sk_q, sk_units;
+    int32_t sk_depth;
+    float *sk_ws;
+};
+
+constexpr int kGroupM = 8;
+constexpr int kXcds = 8;
+constexpr int kSlot = 16;  // k per slot: the depth of one v_mfma_f32_32x32x16_bf16
+
+// min by value: std::min of a kernel argument and a temporary returns a
+// reference the compiler may have to keep in scratch memory.
+__device__ __forceinline__ int64_t imin(int64_t a, int64_t b) { return a < b ? a : b; }
+
+// A pointer that is the same in every lane, in scalar registers.
+__device__ __forceinline__ const float *gt_uniform(const float *p) {
+    const uint64_t u = (uint64_t)p;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
+    return (const float *)((uint64_t)hi << 32 | lo);
+}
+
+struct TileCoord {
+    int64_t batch, m, n;
+};
+
+// Tile t of a launch (t over batch * tiles_m * tiles_n): tiles in groups of
+// kGroupM tile rows, the group's tiles taken down its columns.  In 32 bits: a
+// grid has below 2^31 tiles, and the 64-bit divisions are software loops of
+// some 600 instructions before a block's first load.
+__device__ __forceinline__ TileCoord decode_tile(const GemmArgs &args, uint32_t t) {
+    const uint32_t tm = (uint32_t)args.tiles_m, tn = (uint32_t)args.tiles_n, tiles = tm * tn;
+    TileCoord c;
+    const uint32_t batch = t / tiles;
+    t -= batch * tiles;
+    const uint32_t group_span = (uint32_t)kGroupM * tn;
+    const uint32_t group = t / group_span;
+    const uint32_t first_m = group * kGroupM;
+    const uint32_t gm = tm - first_m < (uint32_t)kGroupM ? tm - first_m : (uint32_t)kGroupM;
+    const uint32_t within = t - group * group_span;
+    // The divisions run on the vector units; back to scalar registers.
+    c.batch = (uint32_t)__builtin_amdgcn_readfirstlane((int)batch);
+    c.m = (uint32_t)__builtin_amdgcn_readfirstlane((int)(first_m + within % gm));
+    c.n = (uint32_t)__builtin_amdgcn_readfirstlane((int)(within / gm));
+    return c;
+}
+
+// Two floats as bf16 pairs h + m + l.  `lost` collects the bits of the last
+// remainders: their low halves are zero exactly where l holds them whole.
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t &h, uint32_t &m, uint32_t &l, uint32_t &lost) {
+    const auto pack = [](float x, float y) {
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector((gt_f2){x, y}, gt_bf2));
+    };
+    const auto lo = [](uint32_t p) { return __uint_as_float(p << 16); };
+    const auto hi = [](uint32_t p) { return __uint_as_float(p & 0xffff0000u); };
+    h = pack(a, b);
+    a -= lo(h);
+    b -= hi(h);
+    m = pack(a, b);
+    a -= lo(m);
+    b -= hi(m);
+    l = pack(a, b);
+    lost |= __float_as_uint(a) | __float_as_uint(b);
+}
+
+// One operand's share of a slot: ROWS rows (of M or N) by 16 k, dealt to the
+// block's lanes in chunks of 8 consecutive k of one row.
+//   KC (k contiguous in memory): a chunk is 32 contiguous bytes, two 16-byte
+//     loads; they need only dword alignment, so any row length will do.
+//   otherwise (rows contiguous): a chunk is 8 loads of one float, each a
+//     whole 256 bytes across the wave (a wave's chunks are 64 rows of one k
+//     half).
+// Either way the lane holds the 8 k that one lane of an MFMA fragment takes,
+// so the pieces are packed in registers and stored as 16 bytes: no transpose,
+// no alignment cases.  In LDS a plane (h, m or l) is kept in fragment order:
+// 32 rows by 16 k are one KiB, chunk (row, half) at 512*half + 16*row, which
+// fragment reads and chunk stores both walk in lane order, free of bank
+// conflicts.
+// Rows past the matrix's edge read its last row (never stored).
+template <int ROWS, int NT, bool KC>
+struct SlotOperand {
+    static constexpr int NC = (ROWS * 2 + NT - 1) / NT;  // chunks per lane
+    static_assert((ROWS * 2) % NT == 0 || NT % (ROWS * 2) == 0, "whole waves share a chunk row");
+    static constexpr int kPlane = ROWS * 2 * kSlot;  // bytes
+    static constexpr int kPitch = ROWS + 32;         // floats per k of the fp32 layout
+    const float *ptr[NC];  // KC: the lane's chunk in the next slot to load; else the operand's first column of it
+    uint32_t voff[NC];     // not KC: the lane's row, in bytes
+    int row[NC], half[NC];
+
+    // base: element (row 0 of the tile, k 0); rows: rows of the matrix from the tile's first on.
+    __device__ __forceinline__ void plan(const float *base, int64_t rows, int64_t ld, unsigned tid) {
+#pragma unroll
+        for (int q = 0; q < NC; q++) {
+            const int c = (int)(tid + q * NT) % (ROWS * 2);
+            if constexpr (KC) {
+                row[q] = (c >> 6) * 32 + (c & 31);
+                half[q] = (c >> 5) & 1;
+            } else {
+                row[q] = c % ROWS;
+                half[q] = __builtin_amdgcn_readfirstlane(c / ROWS);
+            }
+            const int64_t r = row[q] < rows ? row[q] : rows - 1;
+            if constexpr (KC) {
+                ptr[q] = base + r * ld + half[q] * 8;
+            } else {
+                ptr[q] = gt_uniform(base + half[q] * 8 * ld);
+                voff[q] = (uint32_t)(r * 4);
+            }
+        }
+    }
+    __device__ __forceinline__ void advance(int64_t step) {
+#pragma unroll
+        for (int q = 0; q < NC; q++) ptr[q] += step;
+    }
+    // Rows contiguous: one scalar base per k and one 32-bit lane offset.  Both
+    // go through an asm that the compiler cannot see past, since it otherwise
+    // folds the two into a 64-bit lane address per k (16 registers, and
+    // spills).
+    __device__ __forceinline__ static gt_global column(gt_global &p, uint32_t off, int64_t ld) {
+        asm("" : "+s"(p));
+        const gt_global at = (gt_global)((gt_global_bytes)p + off);
+        p += ld;
+        return at;
+    }
+    __device__ __forceinline__ void load(float (&v)[NC][8], int64_t ld) const {
+#pragma unroll
+        for (int q = 0; q < NC; q++) {
+            if constexpr (KC) {
+                const gt_f4u x = *(const gt_f4u *)ptr[q], y = *(const gt_f4u *)(ptr[q] + 4);
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[q][e] = x[e], v[q][4 + e] = y[e];
+            } else {
+                gt_global p = (gt_global)ptr[q];
+                uint32_t off = voff[q];
+                asm("" : "+v"(off));
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[q][e] = *column(p, off, ld);
+            }
+        }
+    }
+    // The first `tail` k of a slot, zero past them (no load is made there).
+    __device__ __forceinline__ void load_tail(float (&v)[NC][8], int64_t ld, int tail) const {
+#pragma unroll
+        for (int q = 0; q < NC; q++) {
+            gt_global p = (gt_global)ptr[q];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                v[q][e] = 0.f;
+                if constexpr (KC) {
+                    if (half[q] * 8 + e < tail) v[q][e] = p[e];
+                } else {
+                    const gt_global at = column(p, voff[q], ld);
+                    if (half[q] * 8 + e < tail) v[q][e] = *at;
+                }
+            }
+        }
+    }
+    __device__ __forceinline__ void store_split(const float (&v)[NC][8], char *lds, uint32_t &lost) const {
+#pragma unroll
+        for (int q = 0; q < NC; q++) {
+            gt_u4 h, m, l;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                uint32_t x, y, z;
+                split_pair(v[q][2 * e], v[q][2 * e + 1], x, y, z, lost);
+                h[e] = x, m[e] = y, l[e] = z;
+            }
+            char *d = lds + (row[q] >> 5) * 1024 + half[q] * 512 + (row[q] & 31) * 16;
+            *(gt_u4 *)d = h;
+            *(gt_u4 *)(d + kPlane) = m;
+            *(gt_u4 *)(d + 2 * kPlane) = l;
+        }
+    }
+    // As floats, [k][row]: the pitch puts k and k + 1 half the banks apart.
+    __device__ __forceinline__ void store_fp32(const float (&v)[NC][8], float *lds) const {
+#pragma unroll
+        for (int q = 0; q < NC; q++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) lds[(half[q] * 8 + e) * kPitch + row[q]] = v[q][e];
+    }
+};
+
+// A BM x BN tile of C on WGM x WGN waves, each (BM/WGM) x (BN/WGN) as 32x32
+// MFMA tiles.  AKC, BKC: the operand is contiguous along k.
+template <int BM, int BN, int WGM, int WGN, bool AKC, bool BKC>
+struct GemmTile {
+    static constexpr int NT = WGM * WGN * 64, WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
+    using OA = SlotOperand<BM, NT, AKC>;
+    using OB = SlotOperand<BN, NT, BKC>;
+    static constexpr int kABytes = 3 * OA::kPlane, kBuf = kABytes + 3 * OB::kPlane;
+    // Three slots in LDS, and the flag of a tile the split does not hold for.
+    static constexpr int kLds = 3 * kBuf + 16;
+    static constexpr int kFp32A = kSlot * OA::kPitch, kFp32Buf = kFp32A + kSlot * OB::kPitch;
+    static_assert(2 * kFp32Buf * 4 <= 3 * kBuf, "the fp32 slots fit the split ones' LDS");
+
+    gt_f16 acc[TM][TN];
+    OA oa;
+    OB ob;
+    char *lds;
+    const GemmArgs &args;
+    int64_t astep, bstep;
+    int lane, wm0, wn0;
+
+    __device__ __forceinline__ GemmTile(const GemmArgs &a, char *l) : lds(l), args(a) {}
+
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+    }
+    __device__ __forceinline__ void load(float (&ra)[OA::NC][8], float (&rb)[OB::NC][8]) const {
+        oa.load(ra, args.lda);
+        ob.load(rb, args.ldb);
+    }
+
+    // `whole` slots from the operands' current pointers on, after the `tail`
+    // k (0: none) behind the last of them.  The partial slot goes first: its
+    // checked loads then fall in the prologue, whose latency is exposed
+    // anyway, and not behind the last whole slot.
+    //
+    // Slot t is computed from one of three LDS buffers while slot t + 2 is split from
+    // registers into another and slot t + 3 is loaded into those
+    // registers.  Slot t + 1's buffer was complete at the barrier before, so the
+    // fragments a slot starts with are read before the barrier that ends the
+    // slot ahead of it.  A wave walks its rows of MFMA tiles; the reads for
+    // the next row, and the slot's splitting and loads, sit among the MFMAs
+    // of the row before.  Loads past the last slot repeat it (a branch around
+    // a load makes the compiler wait for every load at the join).
+    __device__ __forceinline__ uint32_t split_slots(int whole, int tail, unsigned tid, volatile int *bad) {
+        uint32_t lost = 0;
+        float ra[OA::NC][8], rb[OB::NC][8];
+        const int T = whole + (tail ? 1 : 0);
+        int left = whole;  // whole slots not yet loaded
+        const auto next = [&]() {  // load a slot and move on, staying on the last
+            load(ra, rb);
+            left--;
+            oa.advance(left > 0 ? astep : 0);
+            ob.advance(left > 0 ? bstep : 0);
+        };
+        const auto put = [&](int buf) {
+            oa.store_split(ra, lds + buf * kBuf, lost);
+            ob.store_split(rb, lds + buf * kBuf + kABytes, lost);
+        };
+        // After the prologue: every wave is done with the tile before, the flag included.
+        const auto ready = [&]() {
+            __syncthreads();
+            if (tid == 0) *bad = 0;
+        };
+        const char *fa = lds + wm0 * 32 + lane * 16, *fb = lds + kABytes + wn0 * 32 + lane * 16;
+        gt_bf8 A[2][3], B[TN][3];
+        const auto read_a = [&](int buf, int i, gt_bf8 (&d)[3]) {
+#pragma unroll
+            for (int p = 0; p < 3; p++) d[p] = *(const gt_bf8 *)(fa + buf + p * OA::kPlane + i * 1024);
+        };
+        const auto read_b = [&](int buf, int j) {
+#pragma unroll
+            for (int p = 0; p < 3; p++) B[j][p] = *(const gt_bf8 *)(fb + buf + p * OB::kPlane + j * 1024);
+        };
+        // The products (piece of A, piece of B), the smaller first.
+        static constexpr int PA[6] = {2, 1, 1, 0, 0, 0}, PB[6] = {0, 0, 1, 1, 2, 0};
+        int cur = 0, nxt = kBuf, wr = 2 * kBuf;  // this slot's buffer, the next one's, the one being written
+        const auto slot = [&]<bool MORE>() {
+#pragma unroll
+            for (int i = 0; i < TM; i++) {
+                if (i + 1 < TM) read_a(cur, i + 1, A[(i + 1) & 1]);
+                else if (MORE) read_a(nxt, 0, A[TM & 1]);
+#pragma unroll
+                for (int j = 0; j < TN; j++) {
+#pragma unroll
+                    for (int q = 0; q < 6; q++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[i & 1][PA[q]], B[j][PB[q]], acc[i][j], 0, 0, 0);
+                    if (i == TM - 1 && MORE) read_b(nxt, j);
+                }
+                if constexpr (MORE) {
+                    if (i == 0) oa.store_split(ra, lds + wr, lost);
+                    if (i == (TM > 1 ? 1 : 0)) {
+                        oa.load(ra, args.lda);
+                        ob.store_split(rb, lds + wr + kABytes, lost);
+                    }
+                    if (i == (TM > 2 ? 2 : TM - 1)) {
+                        ob.load(rb, args.ldb);
+                        left--;
+                        oa.advance(left > 0 ? astep : 0);
+                        ob.advance(left > 0 ? bstep : 0);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if constexpr (MORE && TM % 2 == 1) {
+#pragma unroll
+                for (int p = 0; p < 3; p++) A[0][p] = A[1][p];
+            }
+            __syncthreads();
+        };
+        const auto first = [&]() {
+            read_a(0, 0, A[0]);
+#pragma unroll
+            for (int j = 0; j < TN; j++) read_b(0, j);
+        };
+        if (tail) {
+            // The partial slot lies `whole` slots on.
+            OA ta = oa;
+            OB tb = ob;
+            ta.advance(whole * astep);
+            tb.advance(whole * bstep);
+            ta.load_tail(ra, args.lda, tail);
+            tb.load_tail(rb, args.ldb, tail);
+            put(0);
+            if (!whole) {
+                ready();
+                first();
+                slot.template operator()<false>();
+                return lost;
+            }
+        } else {
+            next();
+            put(0);
+        }
+        next();
+        put(1);
+        next();
+        ready();
+        first();
+#pragma unroll 1
+        for (int t = 0; t < T; t++) {
+            slot.template operator()<true>();
+            const int c = cur;
+            cur = nxt, nxt = wr, wr = c;
+        }
+        return lost;
+    }
+
+    // The same slots on fp32 MFMA (v_mfma_f32_32x32x2_f32), double-buffered.
+    __device__ __forceinline__ void fp32_slots(int whole, int tail) {
+        float ra[OA::NC][8], rb[OB::NC][8];
+        float *f = (float *)lds;
+        const int T = whole + (tail ? 1 : 0);
+        const auto fetch = [&](int t) {
+            if (t < whole) load(ra, rb);
+            else oa.load_tail(ra, args.lda, tail), ob.load_tail(rb, args.ldb, tail);
+            oa.advance(astep);
+            ob.advance(bstep);
+        };
+        fetch(0);
+        for (int t = 0; t < T; t++) {
+            float *buf = f + (t & 1) * kFp32Buf;
+            oa.store_fp32(ra, buf);
+            ob.store_fp32(rb, buf + kFp32A);
+            if (t + 1 < T) fetch(t + 1);
+            __syncthreads();
+            const float *pa = buf + (lane >> 5) * OA::kPitch + wm0 + (lane & 31);
+            const float *pb = buf + kFp32A + (lane >> 5) * OB::kPitch + wn0 + (lane & 31);
+#pragma unroll 2
+            for (int k = 0; k < kSlot; k += 2) {
+                float x[TM], y[TN];
+#pragma unroll
+                for (int i = 0; i < TM; i++) x[i] = pa[k * OA::kPitch + i * 32];
+#pragma unroll
+                for (int j = 0; j < TN; j++) y[j] = pb[k * OB::kPitch + j * 32];
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int j = 0; j < TN; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i], y[j], acc[i][j], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+    }
+
+    // The tile over its k in [k0, k1) (k1 past the last k: to the end; k0 a
+    // multiple of 16).  Stores it into C, or with `ws` set into
+    // ws[row * BN + column], all of it.  tid: threadIdx.x (the stream-K loop
+    // passes a copy the compiler cannot see through, so that the lane values
+    // are not kept live across tiles).
+    __device__ __forceinline__ void run(TileCoord tc, int64_t k0, int64_t k1, float *ws, unsigned tid) {
+        lane = tid & 63;
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        wm0 = (wave / WGN) * WM;
+        wn0 = (wave % WGN) * WN;
+        const int64_t Kb = args.ktotal ? imin(args.K, args.ktotal - tc.batch * args.K) : args.K;
+        const int64_t m0 = tc.m * BM, n0 = tc.n * BN;
+        const float *A = args.a + tc.batch * args.bsa + (AKC ? m0 * args.lda + k0 : m0 + k0 * args.lda);
+        const float *B = args.b + tc.batch * args.bsb + (BKC ? n0 * args.ldb + k0 : n0 + k0 * args.ldb);
+        astep = AKC ? kSlot : kSlot * args.lda;
+        bstep = BKC ? kSlot : kSlot * args.ldb;
+        const int64_t kspan = imin(k1, Kb) - k0;
+        // 64-bit compares run on the vector units; back to scalar registers.
+        const int whole = __builtin_amdgcn_readfirstlane((int)(kspan >> 4));
+        const int tail = __builtin_amdgcn_readfirstlane((int)(kspan & (kSlot - 1)));
+        volatile int *bad = (volatile int *)(lds + 3 * kBuf);
+        clear();
+        oa.plan(A, args.M - m0, args.lda, tid);
+        ob.plan(B, args.N - n0, args.ldb, tid);
+        const uint32_t lost = split_slots(whole, tail, tid, bad);
+        // A non-finite accumulator leaves a non-finite sum of them.
+        float sum[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) sum[r & 3] += acc[i][j][r];
+        const float s = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+        if ((lost & 0xffffu) != 0 || !(__builtin_fabsf(s) < __builtin_inff())) *bad = 1;
+        __syncthreads();
+        if (__builtin_expect(__builtin_amdgcn_readfirstlane(*bad), 0)) {
+            clear();
+            oa.plan(A, args.M - m0, args.lda, tid);
+            ob.plan(B, args.N - n0, args.ldb, tid);
+            fp32_slots(whole, tail);
+        }
+        // Lane l, register r of a 32x32 tile: row 8*(r/4) + 4*(l/32) + r%4, column l%32.
+        const int rl = 4 * (lane >> 5), cl = lane & 31;
+        if (ws) {
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++)
+                        ws[(wm0 + i * 32 + 8 * (r / 4) + rl + r % 4) * BN + wn0 + j * 32 + cl] = acc[i][j][r];
+            return;
+        }
+        float *C = args.c + tc.batch * args.bsc;
+        const int64_t mrow = m0 + wm0 + rl, ncol = n0 + wn0 + cl;
+        float *cp = C + mrow * args.ldc + ncol;
+        if (m0 + BM <= args.M && n0 + BN <= args.N) {
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    float *p = cp + (int64_t)(i * 32 + 8 * (r / 4) + r % 4) * args.ldc;
+#pragma unroll
+                    for (int j = 0; j < TN; j++) p[j * 32] = acc[i][j][r];
+                }
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int row = i * 32 + 8 * (r / 4) + r % 4;
+                if (mrow + row >= args.M) continue;
+                float *p = cp + (int64_t)row * args.ldc;
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+                    if (ncol + j * 32 < args.N) p[j * 32] = acc[i][j][r];
+            }
+    }
+};
+
+}  // namespace trs

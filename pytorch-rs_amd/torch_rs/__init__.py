@@ -211,7 +211,7 @@ def clone(input: Tensor) -> Tensor:
 
 
 def get_float32_matmul_precision() -> str:
-    """fp32 matmul runs on FP32 MFMA with fp32 accumulation: always "highest"
+    """fp32 matmul keeps fp32 operands and fp32 accumulation: always "highest"
     (python/torch_rs/__init__.py:81-85)."""
     return "highest"
 
