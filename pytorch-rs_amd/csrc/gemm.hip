@@ -12,8 +12,15 @@
 // Three tiles (GemmTile), each in the four operand layouts and at any M, N
 // and K (rows past the edge repeat the last one and are not stored):
 //   256x256  8 waves of 128x64, one block per CU (144 KB of LDS)
-//   128x128  4 waves of 64x64, two blocks per CU
+//   128x128  4 waves of 64x64, or where blocks do not fill the CUs twice 8 of
+//            32x64; two blocks per CU
 //   64x128   4 waves of 32x64, two blocks per CU
+// The 4-wave 128x128 tile reads a third less from LDS per product, which
+// counts where the whole chip runs it and power sets the clock (batched
+// 32x512^3 52.3 us against 54.0, 1000x2047x1500 48.4 against 50.3); the 8-wave
+// one issues its slot in half the instructions per wave, which counts where
+// one block has a CU to itself (200x300x400 12.4 us against 14.6, 700^3 16.6
+// against 18.8, 64^3 6.6 against 8.1).
 // Blocks are remapped so that consecutive tiles share an XCD (each XCD has
 // its own L2), and tiles are walked in groups of kGroupM tile rows.
 #include <hip/hip_runtime.h>
@@ -29,11 +36,13 @@ namespace trs {
 namespace {
 
 template <bool AKC, bool BKC>
-using LargeTile = GemmTile<256, 256, 2, 4, AKC, BKC>;
+using LargeTile = GemmTile<256, 256, 2, 4, 1, AKC, BKC>;
 template <bool AKC, bool BKC>
-using SmallTile = GemmTile<128, 128, 2, 2, AKC, BKC>;
+using SmallTile = GemmTile<128, 128, 2, 2, 2, AKC, BKC>;
 template <bool AKC, bool BKC>
-using MediumTile = GemmTile<64, 128, 2, 2, AKC, BKC>;
+using SmallTile8 = GemmTile<128, 128, 4, 2, 1, AKC, BKC>;
+template <bool AKC, bool BKC>
+using MediumTile = GemmTile<64, 128, 2, 2, 2, AKC, BKC>;
 constexpr int64_t kLarge = 256;
 constexpr int64_t kLargeTileFloats = kLarge * kLarge;
 
@@ -263,12 +272,15 @@ struct GemmPlan {
 };
 
 // One product (or K slice per batch) on a tile, without a split.
-int launch_kind(GemmKind kind, const GemmArgs &g, bool a_plain, bool b_plain, hipStream_t s) {
+int launch_kind(GemmKind kind, const GemmArgs &g, bool a_plain, bool b_plain, int cu_count, hipStream_t s) {
+    const bool alone = (g.M + 127) / 128 * ((g.N + 127) / 128) * g.batch <= cu_count;
     return for_layout(a_plain, b_plain, [&]<bool AKC, bool BKC>() -> int {
         switch (kind) {
         case GemmKind::Large: return launch_tile<LargeTile<AKC, BKC>, 1>(g, kLarge, kLarge, s);
         case GemmKind::Medium: return launch_tile<MediumTile<AKC, BKC>, 2>(g, 64, 128, s);
-        default: return launch_tile<SmallTile<AKC, BKC>, 2>(g, 128, 128, s);
+        default:
+            if (alone) return launch_tile<SmallTile8<AKC, BKC>, 2>(g, 128, 128, s);
+            return launch_tile<SmallTile<AKC, BKC>, 2>(g, 128, 128, s);
         }
     });
 }
@@ -455,7 +467,7 @@ int launch_split_k(const GemmPlan &p, GemmArgs g, bool a_plain, bool b_plain, in
     g.bsb = Ks * sbk;
     g.bsc = mn;
     g.batch = S;
-    rc = launch_kind(p.split_tile, g, a_plain, b_plain, s);
+    rc = launch_kind(p.split_tile, g, a_plain, b_plain, cu_count, s);
     if (rc == TRS_OK) {
         if (mn % 4 == 0 && (uintptr_t)C % 16 == 0) {
             const int64_t n4 = mn / 4;
@@ -595,7 +607,7 @@ int run_peeled(const GemmPlan &p, const GemmSetup &st, int cu_count, hipStream_t
     GemmArgs gm = g;
     gm.M = p.main_m;
     gm.N = p.main_n;
-    TRS_CHECK(launch_kind(GemmKind::Large, gm, st.a_plain, st.b_plain, s));
+    TRS_CHECK(launch_kind(GemmKind::Large, gm, st.a_plain, st.b_plain, cu_count, s));
     if (p.main_m < g.M) {
         SkinnyProblem r;
         r.R = g.M - p.main_m, r.L = g.N, r.K = g.K, r.batch = 1;
@@ -673,16 +685,16 @@ extern "C" int trs_matmul_f32(const float *a, const trs_layout *la, const float 
         rc = launch_stream_k(p, g, st.a_plain, st.b_plain, dev->cu_count, dev->stream);
         if (rc != TRS_E_ALLOCATION_FAILED) return rc;
         // No workspace: run the plan stream-K replaced, unsplit.
-        return launch_kind(p.fallback, g, st.a_plain, st.b_plain, dev->stream);
+        return launch_kind(p.fallback, g, st.a_plain, st.b_plain, dev->cu_count, dev->stream);
     }
     if (p.kind == GemmKind::SplitK) {
         rc = launch_split_k(p, g, st.a_plain, st.b_plain, st.sak, st.sbk, dev->cu_count, dev->stream);
         if (rc != TRS_E_ALLOCATION_FAILED) return rc;
         // No workspace: the split is only an optimisation, so run the tile the
         // plan would otherwise have chosen (nothing was launched).
-        return launch_kind(p.fallback, g, st.a_plain, st.b_plain, dev->stream);
+        return launch_kind(p.fallback, g, st.a_plain, st.b_plain, dev->cu_count, dev->stream);
     }
-    return launch_kind(p.kind, g, st.a_plain, st.b_plain, dev->stream);
+    return launch_kind(p.kind, g, st.a_plain, st.b_plain, dev->cu_count, dev->stream);
 }
 
 extern "C" int trs_matmul_plan_f32(const float *a, const trs_layout *la, const float *b, const trs_layout *lb,

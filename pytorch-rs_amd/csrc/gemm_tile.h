@@ -126,46 +126,48 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t &h, uint32
 }
 
 // One operand's share of a slot: ROWS rows (of M or N) by 16 k, dealt to the
-// block's lanes in chunks of 8 consecutive k of one row.
-//   KC (k contiguous in memory): a chunk is 32 contiguous bytes, two 16-byte
-//     loads; they need only dword alignment, so any row length will do.
-//   otherwise (rows contiguous): a chunk is 8 loads of one float, each a
-//     whole 256 bytes across the wave (a wave's chunks are 64 rows of one k
-//     half).
-// Either way the lane holds the 8 k that one lane of an MFMA fragment takes,
-// so the pieces are packed in registers and stored as 16 bytes: no transpose,
-// no alignment cases.  In LDS a plane (h, m or l) is kept in fragment order:
-// 32 rows by 16 k are one KiB, chunk (row, half) at 512*half + 16*row, which
-// fragment reads and chunk stores both walk in lane order, free of bank
-// conflicts.
+// block's lanes in chunks of CH (8 or 4) consecutive k of one row.
+//   KC (k contiguous in memory): a chunk is one or two 16-byte loads; they
+//     need only dword alignment, so any row length will do.
+//   otherwise (rows contiguous): a chunk is CH loads of one float, each a
+//     whole 256 bytes across the wave (a wave's chunks are 64 rows of the
+//     same k).
+// Either way the lane holds consecutive k of one row, as an MFMA fragment
+// takes them (8 a lane), so the pieces are packed in registers and stored as
+// 8 or 16 bytes: no transpose, no alignment cases.  In LDS a plane (h, m or
+// l) is kept in fragment order: 32 rows by 16 k are one KiB, (row, k) at
+// 512*(k/8) + 16*row + 2*(k%8), which fragment reads walk in lane order, free
+// of bank conflicts.
 // Rows past the matrix's edge read its last row (never stored).
 template <int ROWS, int NT, bool KC>
 struct SlotOperand {
-    static constexpr int NC = (ROWS * 2 + NT - 1) / NT;  // chunks per lane
-    static_assert((ROWS * 2) % NT == 0 || NT % (ROWS * 2) == 0, "whole waves share a chunk row");
+    static constexpr int CH = ROWS * 2 >= NT ? 8 : 4;
+    static constexpr int NC = ROWS * kSlot / CH / NT;  // chunks per lane
+    static_assert(NC >= 1 && NC * NT * CH == ROWS * kSlot && ROWS % 64 == 0, "whole chunks for every lane");
     static constexpr int kPlane = ROWS * 2 * kSlot;  // bytes
     static constexpr int kPitch = ROWS + 32;         // floats per k of the fp32 layout
-    const float *ptr[NC];  // KC: the lane's chunk in the next slot to load; else the operand's first column of it
+    typedef float Regs[NC][CH];
+    const float *ptr[NC];  // KC: the lane's chunk in the next slot to load; else the operand's first row of it
     uint32_t voff[NC];     // not KC: the lane's row, in bytes
-    int row[NC], half[NC];
+    int row[NC], k[NC];    // the chunk's row and first k
 
     // base: element (row 0 of the tile, k 0); rows: rows of the matrix from the tile's first on.
     __device__ __forceinline__ void plan(const float *base, int64_t rows, int64_t ld, unsigned tid) {
 #pragma unroll
         for (int q = 0; q < NC; q++) {
-            const int c = (int)(tid + q * NT) % (ROWS * 2);
+            const int c = (int)(tid + q * NT), l = c & 63;
             if constexpr (KC) {
-                row[q] = (c >> 6) * 32 + (c & 31);
-                half[q] = (c >> 5) & 1;
+                row[q] = c / (32 * kSlot / CH) * 32 + (l & 31);
+                k[q] = ((c >> 6) * 2 + (l >> 5)) % (kSlot / CH) * CH;
             } else {
                 row[q] = c % ROWS;
-                half[q] = __builtin_amdgcn_readfirstlane(c / ROWS);
+                k[q] = __builtin_amdgcn_readfirstlane(c / ROWS * CH);
             }
             const int64_t r = row[q] < rows ? row[q] : rows - 1;
             if constexpr (KC) {
-                ptr[q] = base + r * ld + half[q] * 8;
+                ptr[q] = base + r * ld + k[q];
             } else {
-                ptr[q] = gt_uniform(base + half[q] * 8 * ld);
+                ptr[q] = gt_uniform(base + k[q] * ld);
                 voff[q] = (uint32_t)(r * 4);
             }
         }
@@ -184,67 +186,72 @@ struct SlotOperand {
         p += ld;
         return at;
     }
-    __device__ __forceinline__ void load(float (&v)[NC][8], int64_t ld) const {
+    __device__ __forceinline__ void load(Regs &v, int64_t ld) const {
 #pragma unroll
         for (int q = 0; q < NC; q++) {
             if constexpr (KC) {
-                const gt_f4u x = *(const gt_f4u *)ptr[q], y = *(const gt_f4u *)(ptr[q] + 4);
 #pragma unroll
-                for (int e = 0; e < 4; e++) v[q][e] = x[e], v[q][4 + e] = y[e];
+                for (int e = 0; e < CH; e += 4) {
+                    const gt_f4u x = *(const gt_f4u *)(ptr[q] + e);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) v[q][e + i] = x[i];
+                }
             } else {
                 gt_global p = (gt_global)ptr[q];
                 uint32_t off = voff[q];
                 asm("" : "+v"(off));
 #pragma unroll
-                for (int e = 0; e < 8; e++) v[q][e] = *column(p, off, ld);
+                for (int e = 0; e < CH; e++) v[q][e] = *column(p, off, ld);
             }
         }
     }
     // The first `tail` k of a slot, zero past them (no load is made there).
-    __device__ __forceinline__ void load_tail(float (&v)[NC][8], int64_t ld, int tail) const {
+    __device__ __forceinline__ void load_tail(Regs &v, int64_t ld, int tail) const {
 #pragma unroll
         for (int q = 0; q < NC; q++) {
             gt_global p = (gt_global)ptr[q];
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
+            for (int e = 0; e < CH; e++) {
                 v[q][e] = 0.f;
                 if constexpr (KC) {
-                    if (half[q] * 8 + e < tail) v[q][e] = p[e];
+                    if (k[q] + e < tail) v[q][e] = p[e];
                 } else {
                     const gt_global at = column(p, voff[q], ld);
-                    if (half[q] * 8 + e < tail) v[q][e] = *at;
+                    if (k[q] + e < tail) v[q][e] = *at;
                 }
             }
         }
     }
-    __device__ __forceinline__ void store_split(const float (&v)[NC][8], char *lds, uint32_t &lost) const {
+    __device__ __forceinline__ void store_split(const Regs &v, char *lds, uint32_t &lost) const {
+        typedef uint32_t Pack __attribute__((ext_vector_type(CH / 2)));
 #pragma unroll
         for (int q = 0; q < NC; q++) {
-            gt_u4 h, m, l;
+            Pack h, m, l;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
+            for (int e = 0; e < CH / 2; e++) {
                 uint32_t x, y, z;
                 split_pair(v[q][2 * e], v[q][2 * e + 1], x, y, z, lost);
                 h[e] = x, m[e] = y, l[e] = z;
             }
-            char *d = lds + (row[q] >> 5) * 1024 + half[q] * 512 + (row[q] & 31) * 16;
-            *(gt_u4 *)d = h;
-            *(gt_u4 *)(d + kPlane) = m;
-            *(gt_u4 *)(d + 2 * kPlane) = l;
+            char *d = lds + (row[q] >> 5) * 1024 + (k[q] >> 3) * 512 + (row[q] & 31) * 16 + (k[q] & 7) * 2;
+            *(Pack *)d = h;
+            *(Pack *)(d + kPlane) = m;
+            *(Pack *)(d + 2 * kPlane) = l;
         }
     }
     // As floats, [k][row]: the pitch puts k and k + 1 half the banks apart.
-    __device__ __forceinline__ void store_fp32(const float (&v)[NC][8], float *lds) const {
+    __device__ __forceinline__ void store_fp32(const Regs &v, float *lds) const {
 #pragma unroll
         for (int q = 0; q < NC; q++)
 #pragma unroll
-            for (int e = 0; e < 8; e++) lds[(half[q] * 8 + e) * kPitch + row[q]] = v[q][e];
+            for (int e = 0; e < CH; e++) lds[(k[q] + e) * kPitch + row[q]] = v[q][e];
     }
 };
 
 // A BM x BN tile of C on WGM x WGN waves, each (BM/WGM) x (BN/WGN) as 32x32
-// MFMA tiles.  AKC, BKC: the operand is contiguous along k.
-template <int BM, int BN, int WGM, int WGN, bool AKC, bool BKC>
+// MFMA tiles.  AHEAD slots are on their way from memory in registers (the
+// depth is not what bounds it: 1, 2 and 3 measured within 1%).  AKC, BKC: the operand is contiguous along k.
+template <int BM, int BN, int WGM, int WGN, int AHEAD, bool AKC, bool BKC>
 struct GemmTile {
     static constexpr int NT = WGM * WGN * 64, WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
     using OA = SlotOperand<BM, NT, AKC>;
@@ -273,9 +280,13 @@ struct GemmTile {
 #pragma unroll
                 for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
     }
-    __device__ __forceinline__ void load(float (&ra)[OA::NC][8], float (&rb)[OB::NC][8]) const {
-        oa.load(ra, args.lda);
-        ob.load(rb, args.ldb);
+    struct Slot {  // a slot's floats on their way to LDS
+        typename OA::Regs a;
+        typename OB::Regs b;
+    };
+    __device__ __forceinline__ void load(Slot &r) const {
+        oa.load(r.a, args.lda);
+        ob.load(r.b, args.ldb);
     }
 
     // `whole` slots from the operands' current pointers on, after the `tail`
@@ -293,18 +304,17 @@ struct GemmTile {
     // a load makes the compiler wait for every load at the join).
     __device__ __forceinline__ uint32_t split_slots(int whole, int tail, unsigned tid, volatile int *bad) {
         uint32_t lost = 0;
-        float ra[OA::NC][8], rb[OB::NC][8];
+        Slot in[AHEAD];
         const int T = whole + (tail ? 1 : 0);
         int left = whole;  // whole slots not yet loaded
-        const auto next = [&]() {  // load a slot and move on, staying on the last
-            load(ra, rb);
+        const auto move_on = [&]() {  // staying on the last slot
             left--;
             oa.advance(left > 0 ? astep : 0);
             ob.advance(left > 0 ? bstep : 0);
         };
-        const auto put = [&](int buf) {
-            oa.store_split(ra, lds + buf * kBuf, lost);
-            ob.store_split(rb, lds + buf * kBuf + kABytes, lost);
+        const auto put = [&](const Slot &r, int buf) {
+            oa.store_split(r.a, lds + buf, lost);
+            ob.store_split(r.b, lds + buf + kABytes, lost);
         };
         // After the prologue: every wave is done with the tile before, the flag included.
         const auto ready = [&]() {
@@ -312,6 +322,9 @@ struct GemmTile {
             if (tid == 0) *bad = 0;
         };
         const char *fa = lds + wm0 * 32 + lane * 16, *fb = lds + kABytes + wn0 * 32 + lane * 16;
+        // The products (piece of A, piece of B), the smaller first.
+        static constexpr int PA[6] = {2, 1, 1, 0, 0, 0}, PB[6] = {0, 0, 1, 1, 2, 0};
+        int cur = 0, nxt = kBuf, wr = 2 * kBuf;  // this slot's buffer, the next one's, the one being written
         gt_bf8 A[2][3], B[TN][3];
         const auto read_a = [&](int buf, int i, gt_bf8 (&d)[3]) {
 #pragma unroll
@@ -321,32 +334,31 @@ struct GemmTile {
 #pragma unroll
             for (int p = 0; p < 3; p++) B[j][p] = *(const gt_bf8 *)(fb + buf + p * OB::kPlane + j * 1024);
         };
-        // The products (piece of A, piece of B), the smaller first.
-        static constexpr int PA[6] = {2, 1, 1, 0, 0, 0}, PB[6] = {0, 0, 1, 1, 2, 0};
-        int cur = 0, nxt = kBuf, wr = 2 * kBuf;  // this slot's buffer, the next one's, the one being written
-        const auto slot = [&]<bool MORE>() {
+        // MORE: more slots may follow.  D: the registers holding slot t + 2.
+        const auto slot = [&]<bool MORE, int D>() {
 #pragma unroll
             for (int i = 0; i < TM; i++) {
                 if (i + 1 < TM) read_a(cur, i + 1, A[(i + 1) & 1]);
                 else if (MORE) read_a(nxt, 0, A[TM & 1]);
 #pragma unroll
-                for (int j = 0; j < TN; j++) {
+                for (int q = 0; q < 6; q++)
 #pragma unroll
-                    for (int q = 0; q < 6; q++)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[i & 1][PA[q]], B[j][PB[q]], acc[i][j], 0, 0, 0);
-                    if (i == TM - 1 && MORE) read_b(nxt, j);
-                }
+                    for (int j = 0; j < TN; j++)
+                        acc[i][j] =
+                            __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[i & 1][PA[q]], B[j][PB[q]], acc[i][j], 0, 0, 0);
                 if constexpr (MORE) {
-                    if (i == 0) oa.store_split(ra, lds + wr, lost);
+                    if (i == TM - 1) {
+#pragma unroll
+                        for (int j = 0; j < TN; j++) read_b(nxt, j);
+                    }
+                    if (i == 0) oa.store_split(in[D].a, lds + wr, lost);
                     if (i == (TM > 1 ? 1 : 0)) {
-                        oa.load(ra, args.lda);
-                        ob.store_split(rb, lds + wr + kABytes, lost);
+                        oa.load(in[D].a, args.lda);
+                        ob.store_split(in[D].b, lds + wr + kABytes, lost);
                     }
                     if (i == (TM > 2 ? 2 : TM - 1)) {
-                        ob.load(rb, args.ldb);
-                        left--;
-                        oa.advance(left > 0 ? astep : 0);
-                        ob.advance(left > 0 ? bstep : 0);
+                        ob.load(in[D].b, args.ldb);
+                        move_on();
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -356,61 +368,78 @@ struct GemmTile {
                 for (int p = 0; p < 3; p++) A[0][p] = A[1][p];
             }
             __syncthreads();
+            const int c = cur;
+            cur = nxt, nxt = wr, wr = c;
         };
         const auto first = [&]() {
             read_a(0, 0, A[0]);
 #pragma unroll
             for (int j = 0; j < TN; j++) read_b(0, j);
         };
+        // The first slots' loads all go out together.
+        Slot s0, s1;
         if (tail) {
             // The partial slot lies `whole` slots on.
             OA ta = oa;
             OB tb = ob;
             ta.advance(whole * astep);
             tb.advance(whole * bstep);
-            ta.load_tail(ra, args.lda, tail);
-            tb.load_tail(rb, args.ldb, tail);
-            put(0);
+            ta.load_tail(s0.a, args.lda, tail);
+            tb.load_tail(s0.b, args.ldb, tail);
             if (!whole) {
+                put(s0, 0);
                 ready();
                 first();
-                slot.template operator()<false>();
+                slot.template operator()<false, 0>();
                 return lost;
             }
         } else {
-            next();
-            put(0);
+            load(s0);
+            move_on();
         }
-        next();
-        put(1);
-        next();
+        load(s1);
+        move_on();
+#pragma unroll
+        for (int d = 0; d < AHEAD; d++) {
+            load(in[d]);
+            move_on();
+        }
+        put(s0, 0);
+        put(s1, kBuf);
         ready();
         first();
+        // Slot t takes registers t % AHEAD.
+        const auto upto = [&]<int D>(auto &&self, int n) {
+            if constexpr (D < AHEAD) {
+                if (D < n) {
+                    slot.template operator()<true, D>();
+                    self.template operator()<D + 1>(self, n);
+                }
+            }
+        };
+        int t = 0;
 #pragma unroll 1
-        for (int t = 0; t < T; t++) {
-            slot.template operator()<true>();
-            const int c = cur;
-            cur = nxt, nxt = wr, wr = c;
-        }
+        for (; t + AHEAD <= T; t += AHEAD) upto.template operator()<0>(upto, AHEAD);
+        if constexpr (AHEAD > 1) upto.template operator()<0>(upto, T - t);
         return lost;
     }
 
     // The same slots on fp32 MFMA (v_mfma_f32_32x32x2_f32), double-buffered.
     __device__ __forceinline__ void fp32_slots(int whole, int tail) {
-        float ra[OA::NC][8], rb[OB::NC][8];
+        Slot in;
         float *f = (float *)lds;
         const int T = whole + (tail ? 1 : 0);
         const auto fetch = [&](int t) {
-            if (t < whole) load(ra, rb);
-            else oa.load_tail(ra, args.lda, tail), ob.load_tail(rb, args.ldb, tail);
+            if (t < whole) load(in);
+            else oa.load_tail(in.a, args.lda, tail), ob.load_tail(in.b, args.ldb, tail);
             oa.advance(astep);
             ob.advance(bstep);
         };
         fetch(0);
         for (int t = 0; t < T; t++) {
             float *buf = f + (t & 1) * kFp32Buf;
-            oa.store_fp32(ra, buf);
-            ob.store_fp32(rb, buf + kFp32A);
+            oa.store_fp32(in.a, buf);
+            ob.store_fp32(in.b, buf + kFp32A);
             if (t + 1 < T) fetch(t + 1);
             __syncthreads();
             const float *pa = buf + (lane >> 5) * OA::kPitch + wm0 + (lane & 31);
