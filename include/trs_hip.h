@@ -309,7 +309,8 @@ int trs_matmul_plan_f32(const float *a, const trs_layout *la, const float *b, co
 typedef struct trs_pw_plan_info {
     int32_t variant;    /* 0 nothing to do, 1 flat, 2 rows, 3 transposing, 4 generic */
     int32_t rank;       /* rank after dropping size-1 dims and merging contiguous ones */
-    int32_t vec;        /* 16-byte vector accesses */
+    int32_t vec;        /* 16-byte vector accesses, all of them 16-byte aligned
+                         * (0: at any float, or scalar) */
     int32_t fixed_rank; /* rank the kernel is compiled for (32-bit offsets), 0 = decoded at run time */
     int32_t skew;       /* transposing: a tuple's tiles taken in diagonal order */
     int32_t walk;       /* transposing: outer tuples per block */

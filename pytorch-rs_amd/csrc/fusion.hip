@@ -427,6 +427,13 @@ int resolve_plan_function(Program *prog, DeviceState *dev, const PwPlan &pl, hip
         // The scalar form reads every input plainly, so the streamed mask is
         // not part of its name (one kernel for every mask).
         // Rank 3 fixes the t dim (0 or 1) too; other ranks read it at run time.
+        if (pl.lds) {
+            std::snprintf(name, sizeof name, "trs_fused_xpose_lds_%u_%u", pl.trans, strm);
+            return get_spec_function(prog, dev, name,
+                                     "trs::pw_xpose_lds_body<TrsFused, " + std::to_string(pl.trans) + "u, " +
+                                         std::to_string(strm) + "u>",
+                                     64 * kLdsWaves, fn);
+        }
         const int td = pl.rk == 3 ? (int)pl.g.tdim : -1;
         std::snprintf(name, sizeof name, "trs_fused_xpose_%c%d_%u_%u_%u_%u_%d_%u%s%s", pl.vec ? 'v' : 's', pl.rk,
                       pl.trans, pl.held, pl.once, pl.xbc, pl.walk, pl.vec ? strm : 0u,
@@ -445,8 +452,9 @@ int resolve_plan_function(Program *prog, DeviceState *dev, const PwPlan &pl, hip
 }
 
 // The kernel of a launch plan: looked up by the plan's signature (variant,
-// vector access, role masks, walk, streamed inputs, fixed rank and, at rank
-// 3, the transposing kernel's t dim and plain tiles), resolved on a miss.
+// vector access, role masks, walk, streamed inputs, fixed rank, at rank 3
+// the transposing kernel's t dim and plain tiles, and whether it goes through
+// LDS), resolved on a miss.
 int get_plan_function(Program *prog, DeviceState *dev, const PwPlan &pl, hipFunction_t *fn) {
     // The streamed mask selects among vector kernels only (the scalar
     // transposing kernel ignores it).
@@ -455,7 +463,8 @@ int get_plan_function(Program *prog, DeviceState *dev, const PwPlan &pl, hipFunc
     const uint64_t key = (uint64_t)pl.variant | (uint64_t)pl.vec << 3 | (uint64_t)pl.contig << 4 |
                          (uint64_t)pl.walk << 5 | strm << 9 | (uint64_t)pl.trans << 17 | (uint64_t)pl.held << 25 |
                          (uint64_t)pl.once << 33 | (uint64_t)pl.xbc << 41 | (uint64_t)pl.rk << 49 |
-                         (uint64_t)(pl.rk == 3 ? pl.g.tdim : 0) << 52 | (uint64_t)pl.plain << 53;
+                         (uint64_t)(pl.rk == 3 ? pl.g.tdim : 0) << 52 | (uint64_t)pl.plain << 53 |
+                         (uint64_t)pl.lds << 54;
     {
         std::lock_guard<std::mutex> lock(prog->spec_mu);
         auto it = prog->by_plan[dev->index].find(key);

@@ -787,7 +787,7 @@ int trs_pointwise_plan(int n_inputs, const void *const *inputs, const trs_layout
     info->variant = (int32_t)pl.variant;
     if (pl.variant == PwVariant::Empty) return TRS_OK;
     info->rank = pl.g.rank;
-    info->vec = pl.vec;
+    info->vec = pl.vec && pl.aligned;
     info->fixed_rank = pl.rk;
     info->skew = pl.g.skew;
     info->walk = pl.walk;

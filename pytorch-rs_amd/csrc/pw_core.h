@@ -124,6 +124,10 @@ __device__ __forceinline__ const PwGeom &kernarg_geom() {
 }
 
 typedef float vf4 __attribute__((ext_vector_type(4)));
+// A float4 that may start at any float: global 16-byte accesses need only
+// dword alignment, so rows of any length and views at any offset are read and
+// written as vectors.
+typedef float vf4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint8_t vu8x4 __attribute__((ext_vector_type(4)));
 
 // Output 0 and the inputs; `more` holds outputs 1.. of a multi-output
@@ -165,7 +169,7 @@ __device__ __forceinline__ void ld4(const PwPtrs &p, int64_t off, bool unit, flo
         else q = *src;
         v[0] = (float)q.x; v[1] = (float)q.y; v[2] = (float)q.z; v[3] = (float)q.w;
     } else {
-        const vf4 *src = (const vf4 *)(((const float *)p.in[I]) + off);
+        const vf4u *src = (const vf4u *)(((const float *)p.in[I]) + off);
         vf4 q;
         if constexpr (STREAM) q = __builtin_nontemporal_load(src);
         else q = *src;
@@ -175,7 +179,7 @@ __device__ __forceinline__ void ld4(const PwPtrs &p, int64_t off, bool unit, flo
 
 __device__ __forceinline__ void st4(float *dst, const float *v) {
     vf4 q = {v[0], v[1], v[2], v[3]};
-    __builtin_nontemporal_store(q, (vf4 *)dst);
+    __builtin_nontemporal_store(q, (vf4u *)dst);
 }
 
 // Compile-time loop over inputs.
@@ -298,8 +302,8 @@ __device__ __forceinline__ void decode_outer(const PwGeom &g, int ndims, int64_t
 // ---- pw_flat --------------------------------------------------------------
 // rank 1; ostride 1; istride in {0, 1}.  VEC requires numel % 4 == 0 is NOT
 // assumed: the vector body covers floor(numel/4) groups and a scalar tail the
-// rest.  VEC is chosen by the host only when every unit-stride operand and
-// the output are 16-byte aligned (4-byte for u8).  STRM: bit i set when input
+// rest.  VEC is chosen by the host wherever every float operand is
+// float-aligned and every byte operand 4-byte aligned.  STRM: bit i set when input
 // i is read once (g.streamed), loaded non-temporally.
 template <class F, unsigned U8MASK, bool VEC, unsigned STRM = 0u>
 __device__ __forceinline__ void pw_flat_body(const F &f, const PwGeom &g, const PwPtrs &p) {
@@ -350,7 +354,7 @@ __device__ __forceinline__ void ld4_stream(const PwPtrs &p, int64_t off, float *
         vu8x4 q = __builtin_nontemporal_load((const vu8x4 *)(((const uint8_t *)p.in[I]) + off));
         v[0] = (float)q.x; v[1] = (float)q.y; v[2] = (float)q.z; v[3] = (float)q.w;
     } else {
-        vf4 q = __builtin_nontemporal_load((const vf4 *)(((const float *)p.in[I]) + off));
+        vf4 q = __builtin_nontemporal_load((const vf4u *)(((const float *)p.in[I]) + off));
         v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
     }
 }
@@ -384,7 +388,8 @@ __device__ __forceinline__ void pw_flat_contig_body(const F &f, const PwGeom &g,
 // Innermost dim (size[rank-1] columns) has ostride 1 and istride in {0, 1}.
 // g.rows = product of the outer dims, g.chunks = ceil(cols / chunk) with
 // chunk = g.chunkcols under VEC, else kRowChunk.
-// VEC: cols % 4 == 0 and every unit-stride row start 16-byte aligned.  A lane
+// VEC: at least 4 columns, and any byte operand's rows a multiple of 4 long
+// and 4-byte aligned (float rows may start at any float).  A lane
 // takes one float4 of the row; the block's lanes (g.chunkcols / 4) are
 // chosen per launch for the HBM bytes a block moves (rows_lanes()).
 // STRM: as for pw_flat.
@@ -456,15 +461,17 @@ __device__ __forceinline__ void pw_rows_loop(const F &f, const PwGeom &g, const 
         if constexpr (VEC) {
             const int64_t c0 = chunk * g.chunkcols;
             const int64_t c = c0 + (int64_t)threadIdx.x * 4;
-            // cols % 4 == 0, so a lane's float4 lies wholly inside or past
-            // the row.  Lanes past it load the row's last float4 and store
-            // nothing: no branch around the loads, which would hold back the
-            // geometry reads they depend on until the lane test.  A streamed
+            // Lanes whose float4 ends past the row load the row's last float4:
+            // no branch around the loads, which would hold back the geometry
+            // reads they depend on until the lane test.  Of it they store the
+            // columns from their own on (none, past the row), so that every
+            // output is written once (in place, a second lane would read what
+            // the first had written).  A streamed
             // operand (read once, no broadcast dim) is unit-stride here, so
             // its load kind is fixed at compile time, and the streamed loads
             // are issued first, ahead of the other operands' run-time choice
             // between a vector and a broadcast load.
-            const int64_t cl = c < cols ? c : cols - 4;
+            const int64_t cl = c + 4 <= cols ? c : cols - 4;
             float v[NIN > 0 ? NIN : 1][4];
             static_for<NIN>([&]<int I>() {
                 if constexpr (((STRM >> I) & 1u) != 0u) ld4<U8MASK, I, true>(p, io[I] + cl, true, v[I]);
@@ -474,7 +481,18 @@ __device__ __forceinline__ void pw_rows_loop(const F &f, const PwGeom &g, const 
             });
             float r[NOUT][4];
             eval4(f, v, r);
-            if (c < cols) store4(p, oo + c, r);
+            if (c + 4 <= cols) {
+                store4(p, oo + c, r);
+            } else if (c < cols) {
+#pragma unroll
+                for (int k = 1; k < 4; k++) {
+                    if (cl + k >= c) {
+                        float o[NOUT];
+                        for (int q = 0; q < NOUT; q++) o[q] = r[q][k];
+                        store1<NOUT>(p, oo + cl + k, o);
+                    }
+                }
+            }
         } else {
             const int64_t c0 = chunk * kRowChunk;
             for (int k = 0; k < 4; k++) {
@@ -637,6 +655,18 @@ __device__ __forceinline__ void pw_xpose_body(const F &f, const PwGeom &g, const
         const int64_t t0 = tt * BT, x0 = xt * BX;
         const int64_t t = t0 + (wave % WT) * 32 + 4 * (lane & 7);
         const int64_t x = x0 + (wave / WT) * 32 + 4 * (lane >> 3);
+        // A tile that crosses the edge still loads whole vectors: a lane whose
+        // block ends past it moves the block back to end there (tl, xl) and
+        // stores only its own elements of it.  Scalar, bounds-checked edge
+        // tiles set the pace wherever the sizes leave many of them: (a + b) *
+        // c.mT over [60, 500, 1001], 30% edge tiles.  A byte operand would
+        // lose its 4-byte alignment, so those take the scalar edge, as do
+        // tensors under 4 wide.
+        constexpr bool kClamp = VEC && !PLAIN && U8MASK == 0u;
+        const bool interior = PLAIN || (VEC && t0 + BT <= ts && x0 + BX <= xs);
+        const bool clamped = kClamp && !interior && ts >= 4 && xs >= 4;
+        const int64_t tl = clamped && t + 4 > ts ? ts - 4 : t;
+        const int64_t xl = clamped && x + 4 > xs ? xs - 4 : x;
         // Per-operand lane offset within an outer tuple and the step between
         // its four vectors: along x for TRANS operands (each vector runs along
         // t), along t for the others (each vector runs along x).
@@ -645,18 +675,18 @@ __device__ __forceinline__ void pw_xpose_body(const F &f, const PwGeom &g, const
         Off loff[NIN1], lstep[NIN1];
         static_for<NIN>([&]<int I>() {
             if constexpr ((TRANS >> I) & 1u) {
-                loff[I] = (Off)x * (Off)g.istride[I][xd] + (Off)t;
+                loff[I] = (Off)xl * (Off)g.istride[I][xd] + (Off)tl;
                 lstep[I] = (Off)g.istride[I][xd];
             } else {
-                loff[I] = (Off)t * (Off)g.istride[I][td] + (unit_x.template operator()<I>() ? (Off)x : (Off)0);
+                loff[I] = (Off)tl * (Off)g.istride[I][td] + (unit_x.template operator()<I>() ? (Off)xl : (Off)0);
                 lstep[I] = (Off)g.istride[I][td];
             }
         });
-        const Off ooff_lane = (Off)t * (Off)g.ostride[td] + (Off)x;
-        // The block runs its whole tile with 16-byte vectors when the tile
-        // is interior and the operands aligned (a wave-uniform test), else
-        // every access is scalar and bounds-checked.
-        auto run = [&]<bool FAST, bool ONE_OUTER>() {
+        const Off ooff_lane = (Off)tl * (Off)g.ostride[td] + (Off)xl;
+        // FAST: the block loads its whole tile with 16-byte vectors, else
+        // every access is scalar and bounds-checked.  EDGE: a FAST tile that
+        // crosses the edge (clamped), whose stores are masked.
+        auto run = [&]<bool FAST, bool EDGE, bool ONE_OUTER>() {
             // Operand I's four vectors (raw[j][e]: vector j, element e) at
             // tuple base b.  Element (t+k, x+i) is raw[i][k] for TRANS
             // operands and raw[k][i] for the others.
@@ -726,7 +756,22 @@ __device__ __forceinline__ void pw_xpose_body(const F &f, const PwGeom &g, const
                         for (int q = 0; q < NOUT; q++) r[q][i] = o[q];
                     }
                     const Off ob = ob0 + (Off)k * (Off)g.ostride[td];
-                    if constexpr (FAST) {
+                    if constexpr (FAST && EDGE) {
+                        if (tl + k >= t && t < ts) {
+                            if (xl == x) {
+                                store4(p, ob, r);
+                            } else if (x < xs) {
+#pragma unroll
+                                for (int i = 1; i < 4; i++) {
+                                    if (xl + i >= x) {
+                                        float ov[NOUT];
+                                        for (int q = 0; q < NOUT; q++) ov[q] = r[q][i];
+                                        store1<NOUT>(p, ob + (Off)i, ov);
+                                    }
+                                }
+                            }
+                        }
+                    } else if constexpr (FAST) {
                         store4(p, ob, r);
                     } else if (t + k < ts) {
 #pragma unroll
@@ -779,15 +824,21 @@ __device__ __forceinline__ void pw_xpose_body(const F &f, const PwGeom &g, const
                 compute(v, ocur);
             }
         };
-        const bool fast = PLAIN || (VEC && t0 + BT <= ts && x0 + BX <= xs);
-        if (RK == 3 || g.rank == 3) {
-            if (fast) run.template operator()<true, true>();
-            else run.template operator()<false, true>();
-        } else {
-            if constexpr (RK != 3) {
-                if (fast) run.template operator()<true, false>();
-                else run.template operator()<false, false>();
+        auto pick = [&]<bool ONE_OUTER>() {
+            if constexpr (kClamp) {
+                if (clamped) {
+                    run.template operator()<true, true, ONE_OUTER>();
+                    return;
+                }
             }
+            if (interior) run.template operator()<true, false, ONE_OUTER>();
+            else run.template operator()<false, false, ONE_OUTER>();
+        };
+        if constexpr (RK == 3) {
+            pick.template operator()<true>();
+        } else {
+            if (g.rank == 3) pick.template operator()<true>();
+            else pick.template operator()<false>();
         }
     };
     // The first tile runs outside the loop: a block with one tile ends
@@ -795,6 +846,141 @@ __device__ __forceinline__ void pw_xpose_body(const F &f, const PwGeom &g, const
     // pw_rows, the host launches at most ntiles blocks, so it is unchecked.
     do_tile(blockIdx.x);
     for (int64_t tile = (int64_t)blockIdx.x + gridDim.x; tile < ntiles; tile += gridDim.x) do_tile(tile);
+}
+
+// ---- pw_xpose_lds ---------------------------------------------------------
+// pw_xpose's layouts where the output's rows are not whole 128-byte lines
+// apart and one operand is transposed.  pw_xpose's wave stores 8 rows of 128
+// bytes at a time; off the lines, each of them is two partial lines, and
+// partial writes cost the memory a read each: (a + b) * c.mT over
+// [60, 512, 1001] ran at 2.1 TB/s, over [64, 512, 1024] at 5.5.  Here a block
+// transposes kLdsT x kLdsX (t by x) through LDS, so that a wave stores one row
+// of 1 KiB at a time, 7 whole lines of 9.  Reads are 256-byte runs along t,
+// two 4 x 4 blocks a lane, all issued before any is used.
+// The LDS rows' pitch of 4 floats past 256 keeps the 16-byte stores (4 rows
+// apart, lane to lane) and the row reads on distinct banks.
+constexpr int kLdsT = 64, kLdsX = 256, kLdsPitch = kLdsX + 4, kLdsWaves = 8;
+
+template <class F, unsigned TRANS, unsigned STRM>
+__device__ __forceinline__ void pw_xpose_lds_body(const F &f, const PwGeom &g, const PwPtrs &p) {
+    constexpr int NIN = F::NIN;
+    constexpr int NOUT = nout_of<F>();
+    static_assert(__builtin_popcount(TRANS) == 1, "one transposed operand");
+    constexpr int TI = __builtin_ctz(TRANS);
+    constexpr int STEPS = kLdsX / (16 * kLdsWaves), ROWS = kLdsT / kLdsWaves;
+    __shared__ __attribute__((aligned(16))) float lds[kLdsT * kLdsPitch];
+    const int xd = g.rank - 1, td = g.tdim;
+    const int64_t xs = g.size[xd], ts = g.size[td];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t ntiles = g.groups * g.chunks;
+    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        int64_t c, tt, xt;
+        if (ntiles <= 0xFFFFFFFFll) {
+            const uint32_t q = fast_div((uint32_t)tile, g.fdchunks);
+            const uint32_t rest = (uint32_t)tile - q * g.fdchunks.div;
+            const uint32_t q2 = fast_div(rest, g.fdttiles);
+            c = q;
+            xt = q2;
+            tt = rest - q2 * g.fdttiles.div;
+        } else {
+            c = tile / g.chunks;
+            const int64_t rest = tile - c * g.chunks;
+            tt = rest % g.ttiles;
+            xt = rest / g.ttiles;
+        }
+        // Offsets of the outer tuple c, over the dims other than t and x.
+        int64_t oo = g.ooff, io[NIN];
+        for (int i = 0; i < NIN; i++) io[i] = g.ioff[i];
+        for (int d = xd - 1; d >= 0; d--) {
+            if (d == td) continue;
+            int64_t q, k;
+            if (!g.wide && c < 0x100000000LL) {
+                q = fast_div((uint32_t)c, g.fd[d]);
+                k = (uint32_t)c - (uint32_t)q * g.fd[d].div;
+            } else {
+                q = c / g.size[d];
+                k = c - q * g.size[d];
+            }
+            c = q;
+            oo += k * g.ostride[d];
+            for (int i = 0; i < NIN; i++) io[i] += k * g.istride[i][d];
+        }
+        const int64_t t0 = tt * kLdsT, x0 = xt * kLdsX;
+        // Lane (l, m) takes t0 + 4l .. + 3 of 4 rows of the transposed operand
+        // a step; at the end of t the four are moved back to end there, and
+        // rows past the last read the last (never stored).
+        const int64_t ta = t0 + 4 * (lane & 15), tl = ta + 4 <= ts ? ta : ts - 4;
+        const int xw = 16 * wave + 4 * (lane >> 4);
+        const float *src = (const float *)p.in[TI] + io[TI] + tl;
+        const int64_t xstep = g.istride[TI][xd];
+        vf4 raw[STEPS][4];
+#pragma unroll
+        for (int s = 0; s < STEPS; s++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int64_t x = x0 + xw + s * 16 * kLdsWaves + j;
+                raw[s][j] = *(const vf4u *)(src + (x < xs ? x : xs - 1) * xstep);
+            }
+        // The other operands of this wave's rows, on their way before the
+        // barrier (one latency instead of two); a lane past the row's last
+        // whole float4 reads that one, and takes its elements one by one below.
+        const int64_t x = x0 + 4 * lane;
+        const auto others = [&](int r, float (&v)[NIN][4]) {
+            const int64_t t = t0 + wave * ROWS + r, tc = t < ts ? t : ts - 1;
+            static_for<NIN>([&]<int I>() {
+                if constexpr (I != TI) {
+                    const bool unit = g.istride[I][xd] != 0;
+                    const int64_t at = unit ? (x + 4 <= xs ? x : xs - 4) : 0;
+                    ld4<0u, I, ((STRM >> I) & 1u) != 0u>(p, io[I] + tc * g.istride[I][td] + at, unit, v[I]);
+                }
+            });
+        };
+        constexpr bool kEarly = NIN <= 3;  // more would not fit the registers
+        float v[kEarly ? ROWS : 1][NIN][4];
+        if constexpr (kEarly) {
+#pragma unroll
+            for (int r = 0; r < ROWS; r++) others(r, v[r]);
+        }
+#pragma unroll
+        for (int s = 0; s < STEPS; s++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const vf4 w = {raw[s][0][k], raw[s][1][k], raw[s][2][k], raw[s][3][k]};
+                if (tl + k >= t0) *(vf4 *)&lds[(tl + k - t0) * kLdsPitch + xw + s * 16 * kLdsWaves] = w;
+            }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            const int64_t t = t0 + wave * ROWS + r;
+            if (t >= ts) continue;
+            const float *row = &lds[(wave * ROWS + r) * kLdsPitch + 4 * lane];
+            const int64_t ob = oo + t * g.ostride[td];
+            float(&w)[NIN][4] = v[kEarly ? r : 0];
+            if constexpr (!kEarly) others(r, w);
+            if (x + 4 <= xs) {
+                const vf4 q = *(const vf4 *)row;
+                w[TI][0] = q.x, w[TI][1] = q.y, w[TI][2] = q.z, w[TI][3] = q.w;
+                float o[NOUT][4];
+                eval4(f, w, o);
+                static_for<NOUT>([&]<int O>() {
+                    const vf4 q = {o[O][0], o[O][1], o[O][2], o[O][3]};
+                    *(vf4u *)(out_base<O>(p) + ob + x) = q;
+                });
+            } else {
+                for (int i = 0; i < 4 && x + i < xs; i++) {
+                    float a[NIN];
+                    static_for<NIN>([&]<int I>() {
+                        if constexpr (I == TI) a[I] = row[i];
+                        else a[I] = ld1<0u, I>(p, io[I] + t * g.istride[I][td] + (g.istride[I][xd] != 0 ? x + i : 0));
+                    });
+                    float o[NOUT];
+                    eval1(f, a, o);
+                    store1<NOUT>(p, ob + x + i, o);
+                }
+            }
+        }
+        if (tile + gridDim.x < ntiles) __syncthreads();
+    }
 }
 
 // ---- pw_generic -----------------------------------------------------------

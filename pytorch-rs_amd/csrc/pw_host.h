@@ -32,11 +32,13 @@ constexpr int kMaxSplit = TRS_MAX_RANK - kMaxRank;
 constexpr int kXposeWT = 4, kXposeWX = 2;
 constexpr int kXposeBT = 32 * kXposeWT, kXposeBX = 32 * kXposeWX;
 constexpr int kXposeWalk = 8;  // largest walk: 8, 4 or 2 tuples, dividing the tuple count
+constexpr double kLdsCover = 0.55;
 constexpr int kXposeResident = 4;  // about the pw_xpose blocks (512 lanes) resident per CU
 
 struct PwPlan {
     PwVariant variant = PwVariant::Empty;
-    bool vec = false;
+    bool vec = false;      // 16-byte vector accesses
+    bool aligned = false;  // vec, and every one of them 16-byte aligned (u8: 4-byte)
     bool contig = false;  // Flat + vec with every input unit-stride and read once
     int ntransposed = 0;
     // Xpose: operand role masks (transposed, held over the outer tuples,
@@ -51,6 +53,8 @@ struct PwPlan {
     // Xpose with rk = 3 and vector access: every tile interior and taken in
     // plain order (no diagonal skew), so the kernel tests neither per block.
     bool plain = false;
+    // Xpose: through LDS (pw_xpose_lds), one tuple per block.
+    bool lds = false;
     int nin = 0;
     int block = 256;  // lanes per block (kFlatBlock for the flat variants)
     int64_t grid = 0;
@@ -311,8 +315,15 @@ inline int plan_pointwise(const trs_layout *lo, float *out, int nin, const void 
         if (!bcast) g.streamed |= 1u << i;
     }
 
-    // Alignment of a unit-stride access along dim `ud` for operand bytes, in
-    // every part of a split launch (`sst`: the operand's split-dim strides).
+    // Vectors start at any element of a float operand; a byte operand's four
+    // must be 4-byte aligned, which with rows (or, transposed, columns) moved
+    // back at an edge takes a multiple of 4 of them.
+    auto vector_ok = [&](const void *base, bool is_aligned, int64_t length, int eb) {
+        return eb == 4 ? (uintptr_t)base % 4 == 0 : is_aligned && length % 4 == 0;
+    };
+    // 16-byte alignment (4-byte for u8) of a unit-stride access along dim
+    // `ud` for operand bytes, in every part of a split launch (`sst`: the
+    // operand's split-dim strides).
     auto aligned = [&](const void *base, int64_t off, const int64_t *strides, const int64_t *sst, int ud, int eb) {
         const uint64_t addr = (uint64_t)(uintptr_t)base + (uint64_t)off * (uint64_t)eb;
         if (addr % (uint64_t)(4 * eb) != 0) return false;
@@ -343,15 +354,26 @@ inline int plan_pointwise(const trs_layout *lo, float *out, int nin, const void 
             if (last(g.ioff[i], is[i], plan->sis[i]) > (int64_t)UINT32_MAX) return false;
         return true;
     };
+    auto outputs_float_aligned = [&]() {
+        bool ok = (uintptr_t)out % 4 == 0;
+        for (int o = 1; o < nout; o++) ok = ok && (uintptr_t)more[o - 1] % 4 == 0;
+        return ok;
+    };
     bool unit_or_bcast = os[inner] == 1;
     for (int i = 0; i < nin; i++) unit_or_bcast &= is[i][inner] == 0 || is[i][inner] == 1;
     const int64_t cap = g_pw_grid_cap.load(std::memory_order_relaxed);
     const int64_t want = cap > 0 ? cap : kMaxGrid;
 
     if (unit_or_bcast) {
-        bool vec = outputs_aligned();
+        plan->aligned = outputs_aligned();
+        bool vec = outputs_float_aligned();
         for (int i = 0; i < nin; i++)
-            if (is[i][inner] == 1) vec &= aligned(bases[i], g.ioff[i], is[i], plan->sis[i], inner, elem_bytes[i]);
+            if (is[i][inner] == 1) {
+                const bool al = aligned(bases[i], g.ioff[i], is[i], plan->sis[i], inner, elem_bytes[i]);
+                plan->aligned &= al;
+                // The flat kernels' tail is scalar: any length.
+                vec &= vector_ok(bases[i], al, rank == 1 ? 0 : size[inner], elem_bytes[i]);
+            }
         if (rank == 1) {
             plan->variant = PwVariant::Flat;
             plan->vec = vec;
@@ -363,7 +385,8 @@ inline int plan_pointwise(const trs_layout *lo, float *out, int nin, const void 
             plan->grid = std::min<int64_t>(std::max<int64_t>(1, (work + kFlatBlock - 1) / kFlatBlock), want);
         } else {
             plan->variant = PwVariant::Rows;
-            plan->vec = vec && size[inner] % 4 == 0;
+            plan->vec = vec && size[inner] >= 4;
+            plan->aligned &= size[inner] % 4 == 0;
             plan->block = plan->vec ? rows_lanes(g.streamed, nin, elem_bytes, nout) : 256;
             g.chunkcols = plan->vec ? 4 * plan->block : 0;
             g.rows = numel / size[inner];
@@ -395,13 +418,15 @@ inline int plan_pointwise(const trs_layout *lo, float *out, int nin, const void 
         if (ok && tdim >= 0) {
             g.tdim = tdim;
             g.transposed = tmask;
-            bool vec = outputs_aligned();
+            plan->aligned = outputs_aligned();
+            bool vec = outputs_float_aligned();
             for (int i = 0; i < nin; i++) {
-                if ((tmask >> i) & 1u) {
-                    vec &= aligned(bases[i], g.ioff[i], is[i], plan->sis[i], tdim, elem_bytes[i]);
-                } else if (is[i][inner] == 1) {
-                    vec &= aligned(bases[i], g.ioff[i], is[i], plan->sis[i], inner, elem_bytes[i]);
-                }
+                const int ud = (tmask >> i) & 1u ? tdim : inner;
+                if (is[i][ud] != 1) continue;
+                const bool al = aligned(bases[i], g.ioff[i], is[i], plan->sis[i], ud, elem_bytes[i]);
+                plan->aligned &= al;
+                // Byte operands' edge tiles are scalar (pw_xpose_body): any length.
+                vec &= vector_ok(bases[i], al, 0, elem_bytes[i]);
             }
             plan->vec = vec;
             plan->ntransposed = nt;
@@ -419,6 +444,31 @@ inline int plan_pointwise(const trs_layout *lo, float *out, int nin, const void 
                     if (outer_zero) plan->held |= 1u << i;
                     else if (is[i][tdim] == 0) plan->once |= 1u << i;
                 }
+            }
+            // Through LDS where the output's rows are not whole lines apart, the
+            // one transposed operand and every other are floats, and the 64 x
+            // 256 tiles are at least kLdsCover full.  Fused (a + b) * c.mT,
+            // through LDS against the direct tiles, in us: [60, 500, 1001] 62 /
+            // 119, [20, 1023, 999] 49 / 78, [16, 64, 300] (0.59 full) 7.0 /
+            // 10.6; emptier tiles lose: [33, 77, 901] (0.53) 11.4 / 8.8, [10,
+            // 300, 130] (0.24) 9.3 / 5.5.
+            bool whole_lines = true, floats = true;
+            for (int d = 0; d < inner; d++) whole_lines &= os[d] % 32 == 0;
+            for (int i = 0; i < nin; i++) floats &= elem_bytes[i] == 4;
+            const auto cover = [](int64_t n, int64_t tile) { return (double)n / (double)((n + tile - 1) / tile * tile); };
+            if (vec && nt == 1 && floats && !whole_lines && size[tdim] >= 4 && size[inner] >= 4 &&
+                cover(size[tdim], kLdsT) * cover(size[inner], kLdsX) >= kLdsCover) {
+                plan->lds = true;
+                plan->held = plan->once = plan->xbc = 0;
+                g.groups = g.rows;
+                g.ttiles = (size[tdim] + kLdsT - 1) / kLdsT;
+                g.chunks = g.ttiles * ((size[inner] + kLdsX - 1) / kLdsX);
+                const bool small = g.groups * g.chunks <= (int64_t)UINT32_MAX;
+                g.fdchunks = make_fast_div(small ? (uint32_t)g.chunks : 1u);
+                g.fdttiles = make_fast_div(small ? (uint32_t)g.ttiles : 1u);
+                plan->block = 64 * kLdsWaves;
+                plan->grid = std::min<int64_t>(g.groups * g.chunks, want);
+                return TRS_OK;
             }
             // When an operand is held, each block walks the largest of 8, 4
             // or 2 tuples that divides the tuple count (the held operand is

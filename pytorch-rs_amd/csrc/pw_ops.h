@@ -104,6 +104,10 @@ template <class F, unsigned M, bool V, unsigned TR, unsigned S>
 __global__ void __launch_bounds__(64 * kXposeWT * kXposeWX) k_xpose(PwGeom, PwPtrs p, F f) {
     pw_xpose_body<F, M, V, kXposeWT, kXposeWX, TR, 0u, 0u, 1, S>(f, kernarg_geom(), p);
 }
+template <class F, unsigned TR>
+__global__ void __launch_bounds__(64 * kLdsWaves) k_xpose_lds(PwGeom, PwPtrs p, F f) {
+    pw_xpose_lds_body<F, TR, 0u>(f, kernarg_geom(), p);
+}
 template <class F, unsigned M>
 __global__ void __launch_bounds__(kGenericBlock) k_generic(PwGeom, PwPtrs p, F f) { pw_generic_body<F, M>(f, kernarg_geom(), p); }
 
@@ -155,6 +159,12 @@ int launch_part(const F &f, const PwPlan &pl, const PwGeom &g, hipStream_t s) {
         // One outer tuple per block (no roles): every transposed-operand mask.
         with_mask<NIN>(pl.trans, [&]<unsigned TR>() {
             if constexpr (TR != 0u) {
+                if constexpr (M == 0u && __builtin_popcount(TR) == 1) {
+                    if (pl.lds) {
+                        hipLaunchKernelGGL((k_xpose_lds<F, TR>), grid, block, 0, s, g, pl.p, f);
+                        return;
+                    }
+                }
                 if (pl.vec)
                     with_mask<NIN>(sm, [&]<unsigned S>() {
                         hipLaunchKernelGGL((k_xpose<F, M, true, TR, S>), grid, block, 0, s, g, pl.p, f);
