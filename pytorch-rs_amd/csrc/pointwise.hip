@@ -184,7 +184,10 @@ __global__ void __launch_bounds__(kHelperLanes) reduce_bcast_kernel(const float 
 // chain costs R dependent adds whatever the layout (about 6 cycles each for a
 // wave fed from LDS).
 //
-// A block owns 32 chains.  Eight producer waves load stages of SR rows of
+// A block owns 32 chains (at the right edge of a KI that is no multiple of
+// that, quads of chains are moved back to end at KI: a chain is then added by
+// two lanes, alike, and stored by the one whose own it is).  Eight producer
+// waves load stages of SR rows of
 // those 32 columns AHEAD stages in advance into registers: each lane SR/256
 // blocks of 4x4 (4 rows of 4 chains), multiplied by `other` (one rounding, as
 // the reference's up * other), transposed in registers and stored
@@ -261,16 +264,25 @@ __global__ void __launch_bounds__(kStLanes) reduce_stage_kernel(const float *up,
     __shared__ __attribute__((aligned(16))) float stage[2][CH][PITCH];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    const int64_t groups = g.KI / CH;
+    const int64_t groups = (g.KI + CH - 1) / CH;
     const int64_t ko = blockIdx.x / groups;
     int64_t gi = blockIdx.x % groups;
     if (CH == 16 && groups % 16 == 0)  // blocks b, b + 8: the two halves of one 128 B line
         gi = (gi / 16) * 16 + 2 * (gi % 8) + (gi / 8) % 2;
     const int64_t ki0 = gi * CH;
+    // The block's first column in memory and the columns it reads from there.
+    const int64_t cb = g.KI >= CH ? (ki0 < g.KI - CH ? ki0 : g.KI - CH) : 0;
+    const int width = g.KI < CH ? (int)g.KI : CH;
+    // Chain quad q's first column past cb.
+    const auto quad_col = [&](int q) {
+        const int64_t c = ki0 + q * 4;
+        return (int)((c < g.KI - 4 ? c : g.KI - 4) - cb);
+    };
     const int64_t nst = (g.R + SR - 1) / SR;
     const int64_t nit = (nst + AHEAD - 1) / AHEAD * AHEAD;  // stages run, padded to whole rings
     if (wave < kStProducers) {
-        const int cq = lane / RQ;  // chains cq*4 .. cq*4+3
+        const int cq = lane / RQ;  // chains cq*4 .. cq*4+3 of the stage
+        const int cs = quad_col(cq);
         // row quads j*QUADS + wave*RQ + lane%RQ of a stage, j < NQ
         const int quad0 = wave * RQ + lane % RQ;
         // Loads go through a buffer descriptor per stage, built in scalar
@@ -278,18 +290,18 @@ __global__ void __launch_bounds__(kStLanes) reduce_stage_kernel(const float *up,
         // offsets within a stage never change, and the descriptor's extent
         // ends after the last row below R, so the hardware returns 0 for the
         // rows past R (never added) without any per-row address arithmetic.
-        const float *ub = up + ko * g.up_ko + ki0;
-        const float *ob = OT != kOtNone ? other + g.other_off + ko * g.ot_ko + ki0 * g.ot_ki : nullptr;
+        const float *ub = up + ko * g.up_ko + cb;
+        const float *ob = OT != kOtNone ? other + g.other_off + ko * g.ot_ko + cb * g.ot_ki : nullptr;
         int vu[NQ][4], vo[NQ][4];
 #pragma unroll
         for (int j = 0; j < NQ; j++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int64_t row = (j * QUADS + quad0) * 4 + i;
-                vu[j][i] = (int)((row * g.up_r + cq * 4) * 4);
-                if constexpr (OT == kOtVecKi) vo[j][i] = (int)((row * g.ot_r + cq * 4) * 4);
+                vu[j][i] = (int)((row * g.up_r + cs) * 4);
+                if constexpr (OT == kOtVecKi) vo[j][i] = (int)((row * g.ot_r + cs) * 4);
                 else if constexpr (OT == kOtVecR)
-                    vo[j][i] = (int)(((int64_t)(cq * 4 + i) * g.ot_ki + (j * QUADS + quad0) * 4) * 4);
+                    vo[j][i] = (int)(((int64_t)(cs + i) * g.ot_ki + (j * QUADS + quad0) * 4) * 4);
                 else vo[j][i] = 0;
             }
         // ru[s][j][i]: row i's 4 chains; ro[s][j][i]: the same for kOtVecKi
@@ -298,26 +310,26 @@ __global__ void __launch_bounds__(kStLanes) reduce_stage_kernel(const float *up,
         auto issue = [&](int slot, int64_t st) {
             const int64_t sc = st < nst ? st : nst - 1;  // past the end: no rows, base kept in range
             const int64_t rem = g.R - st * SR;            // rows from this stage's first on
-            const auto rs = stage_rsrc(ub + sc * SR * g.up_r, stage_span(rem, g.up_r, CH));
+            const auto rs = stage_rsrc(ub + sc * SR * g.up_r, stage_span(rem, g.up_r, width));
 #pragma unroll
             for (int j = 0; j < NQ; j++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) ru[slot][j][i] = buffer_vf4(rs, vu[j][i]);
             if constexpr (OT == kOtVecKi) {
-                const auto os = stage_rsrc(ob + sc * SR * g.ot_r, stage_span(rem, g.ot_r, CH));
+                const auto os = stage_rsrc(ob + sc * SR * g.ot_r, stage_span(rem, g.ot_r, width));
 #pragma unroll
                 for (int j = 0; j < NQ; j++)
 #pragma unroll
                     for (int i = 0; i < 4; i++) ro[slot][j][i] = buffer_vf4(os, vo[j][i]);
             } else if constexpr (OT == kOtVecR) {
                 // the last chain's remaining rows end the extent
-                const auto os = stage_rsrc(ob + sc * SR, stage_span(rem, 1, (CH - 1) * g.ot_ki + 1));
+                const auto os = stage_rsrc(ob + sc * SR, stage_span(rem, 1, (width - 1) * g.ot_ki + 1));
 #pragma unroll
                 for (int j = 0; j < NQ; j++)
 #pragma unroll
                     for (int i = 0; i < 4; i++) ro[slot][j][i] = buffer_vf4(os, vo[j][i]);
             } else if constexpr (OT == kOtScalar) {
-                const float *oc = ob + cq * 4 * g.ot_ki;
+                const float *oc = ob + cs * g.ot_ki;
 #pragma unroll
                 for (int j = 0; j < NQ; j++)
 #pragma unroll
@@ -397,7 +409,29 @@ __global__ void __launch_bounds__(kStLanes) reduce_stage_kernel(const float *up,
                     for (int q = 0; q < 8; q++) a[q] = b[q];
                 }
             } else {
-                for (int64_t r = 0; r < left; r++) acc += row[r];
+                // A last, partial stage: whole groups of 32 rows, quads, rows.
+                const int n = (int)left;
+                int r = 0;
+                for (; r + 32 <= n; r += 32) {
+                    vf4 a[8];
+#pragma unroll
+                    for (int q = 0; q < 8; q++) a[q] = *(const vf4 *)&row[r + q * 4];
+#pragma unroll
+                    for (int q = 0; q < 8; q++) {
+                        acc += a[q][0];
+                        acc += a[q][1];
+                        acc += a[q][2];
+                        acc += a[q][3];
+                    }
+                }
+                for (; r + 4 <= n; r += 4) {
+                    const vf4 a = *(const vf4 *)&row[r];
+                    acc += a[0];
+                    acc += a[1];
+                    acc += a[2];
+                    acc += a[3];
+                }
+                for (; r < n; r++) acc += row[r];
             }
         };
         for (int64_t it = -AHEAD; it < nit; it++) {
@@ -405,7 +439,10 @@ __global__ void __launch_bounds__(kStLanes) reduce_stage_kernel(const float *up,
             __syncthreads();
         }
         if (nit == nst && active) add_stage(nst - 1);  // written before the last barrier
-        if (active) grad[ko * g.KI + ki0 + lane] = acc;
+        // The chain this lane added, stored where it is the lane's own.
+        const int64_t chain = cb + quad_col((lane & (CH - 1)) >> 2) + (lane & 3);
+        const int64_t own = ki0 + ((lane & (CH - 1)) & ~3);
+        if (active && chain >= own && own < g.KI) grad[ko * g.KI + chain] = acc;
     }
 }
 
@@ -464,6 +501,30 @@ bool reduce_cols_plan(const ReduceGeom &rg, bool has_other, RedColsGeom *cg) {
     cg->ot_ki = oki;
     cg->other_off = rg.other_off;
     return true;
+}
+
+// Whether the staged kernel is the faster one for cg's chains: up to a number
+// of chains that grows with their length.  A staged block costs about 4.5 us
+// whatever its rows, and its blocks run in rounds; the unrolled kernel costs a
+// memory latency per 8 rows, with any number of chains, until it is bound by
+// memory.  Measured, staged / unrolled, in us:
+//   rows   chains per CU
+//     16   32: 5.4 / 6.7      64: 7.4 / 6.6
+//     64   64: 7.6 / 7.8     128: 11.7 / 8.1
+//    128  128: 13.8 / 15.3   256: 23.1 / 15.6
+//    255  128: 19.9 / 28.0   256: 34.1 / 28.3
+//    400  256: 38.7 / 50.3   512: 72.0 / 57.5
+//   1000  256: 77.3 / 123    512: 147 / 138
+// Chains that start and stay 16-byte aligned, in whole blocks, read faster
+// ([1000, 65536] 64 us): staged from 256 rows on, whatever their number.
+// (A gradient [8192, 1000] -> [1000] took 796 us unrolled, 32.6 staged.)
+constexpr int64_t kStMinRows = 16;
+
+bool staged_pays(const RedColsGeom &cg, bool whole_aligned, int cu_count) {
+    if (cg.R < kStMinRows) return false;
+    if (whole_aligned && cg.R >= kStRows) return true;
+    const int64_t per_cu = cg.R < 64 ? 32 : cg.R < 128 ? 64 : cg.R < 256 ? 128 : cg.R < 512 ? 256 : 448;
+    return cg.KO * cg.KI <= per_cu * cu_count;
 }
 
 int reduce_to_operand(const float *up, const trs_layout *lout, const float *other,
@@ -546,29 +607,31 @@ int reduce_to_operand(const float *up, const trs_layout *lout, const float *othe
         TRS_LAUNCH_CHECK("fill kernel");
         return TRS_OK;
     }
-    // The staged kernel: reduced dims merging into at least one full stage
-    // of rows, kept dims merging into an outer and an inner part whose up
-    // stride is 1 and whose size is a multiple of 32, 16-byte aligned.
-    // Byte offsets within a stage are 32-bit: (256 * stride + 32) * 4 must
-    // stay below 2^31 for each operand read through a descriptor.
+    // The staged kernel: kept dims merging into an outer and an inner part of
+    // at least 4 whose up stride is 1, and chains long enough for their number
+    // (kStMinRows).  Its 16-byte loads need only dword alignment.  Byte
+    // offsets within a stage are 32-bit: (256 * stride + 32) * 4 must stay
+    // below 2^31 for each operand read through a descriptor.
     auto fits = [](int64_t extent) { return extent >= 0 && extent * 4 < (int64_t)INT32_MAX; };
     RedColsGeom cg{};
-    if (reduce_cols_plan(rg, other != nullptr, &cg) && cg.R >= kStRows && cg.KI % kStChains == 0 &&
-        cg.KO * (cg.KI / kStChains) <= INT32_MAX && (uintptr_t)up % 16 == 0 && cg.up_ko % 4 == 0 &&
-        cg.up_r % 4 == 0 && fits(kStRows * cg.up_r + kStChains) &&
+    const auto blocks_of = [&](int64_t ch) { return cg.KO * ((cg.KI + ch - 1) / ch); };
+    if (reduce_cols_plan(rg, other != nullptr, &cg) && cg.KI >= 4 &&
+        staged_pays(cg, (uintptr_t)up % 16 == 0 && cg.up_ko % 4 == 0 && cg.up_r % 4 == 0 && cg.KI % kStChains == 0,
+                    dev->cu_count) &&
+        blocks_of(16) <= INT32_MAX && (uintptr_t)up % 4 == 0 && fits(kStRows * cg.up_r + kStChains) &&
+        (!other || (uintptr_t)other % 4 == 0) &&
         (!other || (cg.ot_ko >= 0 && cg.ot_r >= 0 && cg.ot_ki >= 0))) {
         auto launch = [&]<int CH, int SR>() {
-            const int64_t grid = cg.KO * (cg.KI / CH);
+            const int64_t grid = blocks_of(CH);
             const dim3 gd((unsigned)grid), bd(kStLanes);
             if (!other) {
                 hipLaunchKernelGGL((reduce_stage_kernel<kOtNone, 2, SR, CH>), gd, bd, 0, dev->stream, up, other, cg,
                                    grad);
             } else {
-                const bool base16 = (uintptr_t)(other + cg.other_off) % 16 == 0 && cg.ot_ko % 4 == 0;
-                if (base16 && cg.ot_ki == 1 && cg.ot_r % 4 == 0 && fits(SR * cg.ot_r + CH))
+                if (cg.ot_ki == 1 && fits(SR * cg.ot_r + CH))
                     hipLaunchKernelGGL((reduce_stage_kernel<kOtVecKi, 2, SR, CH>), gd, bd, 0, dev->stream, up, other,
                                        cg, grad);
-                else if (base16 && cg.ot_r == 1 && cg.ot_ki % 4 == 0 && cg.R % 4 == 0 && fits(CH * cg.ot_ki + SR))
+                else if (cg.ot_r == 1 && cg.R % 4 == 0 && fits(CH * cg.ot_ki + SR))
                     hipLaunchKernelGGL((reduce_stage_kernel<kOtVecR, 2, SR, CH>), gd, bd, 0, dev->stream, up, other,
                                        cg, grad);
                 else
@@ -578,7 +641,7 @@ int reduce_to_operand(const float *up, const trs_layout *lout, const float *othe
         };
         // 16-chain blocks with 512-row stages when 32-chain blocks would
         // leave CUs idle (a bias gradient over [8192, 4096]: 128 blocks).
-        if (cg.KO * (cg.KI / kStChains) < dev->cu_count && cg.R >= 2 * kStRows && fits(2 * kStRows * cg.up_r + 16))
+        if (blocks_of(kStChains) < dev->cu_count && cg.R >= 2 * kStRows && fits(2 * kStRows * cg.up_r + 16))
             launch.template operator()<16, 2 * kStRows>();
         else
             launch.template operator()<kStChains, kStRows>();
