@@ -64,7 +64,7 @@ __global__ void __launch_bounds__(T::NT, MINB) gemm_split_tile(GemmArgs args) {
         bid = (bid % kXcds) * per_xcd + bid / kXcds;
     }
     T tile(args, lds);
-    tile.run(decode_tile(args, bid), 0, INT64_MAX, nullptr, threadIdx.x);
+    tile.template run<true>(decode_tile(args, bid), 0, INT64_MAX, nullptr, threadIdx.x);
 }
 
 // Stream-K: one persistent block per CU, block b taking the (tile, slice)
@@ -89,7 +89,7 @@ __global__ void __launch_bounds__(T::NT, 1) gemm_split_tile_sk(GemmArgs args) {
         unsigned tid = threadIdx.x;
         asm volatile("" : "+v"(tid));
         T tile(args, lds);
-        tile.run(decode_tile(args, (uint32_t)t), qb * args.sk_depth, qe * args.sk_depth, ws, tid);
+        tile.template run<false>(decode_tile(args, (uint32_t)t), qb * args.sk_depth, qe * args.sk_depth, ws, tid);
         u += qe - qb;
     }
 }

@@ -5,17 +5,29 @@
 // h = rn(x), m = rn(x - h), l = x - h - m (bf16 has 8 significant bits and
 // float's exponent range, so nothing is scaled).  Of the nine products of
 // two such sums the six of weight 2^-16 and above are computed, each exact in
-// the matrix cores, and added into one fp32 accumulator, the small ones
-// first; the three left out are below 2^-24 of |x||y| together.  bf16 MFMA
-// runs 16 times the rate of fp32 MFMA, so six products cost 3/8 of the fp32
-// instruction's time.  Rounding to nearest matters: with truncated pieces
-// every small product has the sign of the whole one, and the accumulator's
-// alignment loses them in one direction (K = 4096 on positive data: 9.5e-6).
+// the matrix cores and added in fp32, the small ones first; the three left
+// out are below 2^-24 of |x||y| together.  bf16 MFMA runs 16 times the rate of
+// fp32 MFMA, so six products cost 3/8 of the fp32 instruction's time.
+// Rounding to nearest matters: with truncated pieces every small product has
+// the sign of the whole one, and the accumulator's alignment loses them in
+// one direction (K = 4096 on positive data: 9.5e-6).
 //
-// Error against 64 bits (2-norm, relative; development probe, fp32 MFMA on
-// the same inputs in brackets): N(0,1) K = 16 3.3e-8 (7.4e-8), K = 256
-// 2.4e-7 (2.9e-7), K = 4096 1.01e-6 (1.15e-6); |N(0,1)| K = 4096 6.2e-7
-// (9.9e-7).
+// The matrix core rounds the accumulator once per 8 k, so six products of 16 k
+// round it 12 times where fp32 MFMA does 8.  So each MFMA tile takes the five
+// small products of every other slot in a sum of their own (`low`) and adds
+// that once: 3 roundings there, 7.5 on average.  Half the MFMA tiles do it in
+// one slot and the other half in the next, which spreads the adds.  In every
+// slot for every tile it halves the error again, at 634 us for 4096^3; not at
+// all, operands with many zeros (a relu's output), which fp32 MFMA adds without
+// rounding, have up to 1.2 times its error (565 us); this way 593 us.
+//
+// Error against 64 bits (2-norm over sqrt of the sum of squares; the fp32 MFMA
+// tiles this replaced on the same inputs in brackets), [1000, K] @ [K, 1000]
+// of relu(N(0,1)) and U(-1, 1)/sqrt(K): K = 64 8.6e-8 (1.05e-7), K = 512
+// 1.30e-7 (1.50e-7), K = 2048 1.86e-7 (2.1e-7), K = 6144 2.31e-7 (2.58e-7),
+// K = 16384 3.8e-7 (4.1e-7); N(0,1) and |N(0,1)| are further below.  Of the
+// training step [2048,1024] -> 1500 -> 512: out 3.1e-7, dX 2.5e-7, dW1
+// 2.2e-7, dW2 5.9e-8 (6.9e-8 to 7.2e-8).
 //
 // Where the split does not hold -- a value whose lowest bits fall below
 // bf16's smallest subnormal (|x| < 2^-110 with low bits set), an infinity, a
@@ -23,10 +35,11 @@
 // MFMA (fp32_slots): the split notes lost bits as it goes, and everything
 // else leaves a non-finite accumulator.
 //
-// What bounds it: the card's power.  At 4096^3 a tile of zeros runs 416 us
-// (1,980 TFLOP/s of bf16), random values 570 us (1,445) at a lower clock; the
-// MFMAs alone on random values 466 us, with their LDS reads 490, with the
-// global loads 540.  The fp32 MFMA kernel this replaced took 945 us.
+// What bounds it: the card's power.  At 4096^3 random values run 593 us
+// (1,390 TFLOP/s of bf16).  With every product added straight to the
+// accumulator a product of zeros ran 416 us (1,980 TFLOP/s) and random values
+// 570 us at a lower clock: the MFMAs alone 466 us, with their LDS reads 490, with
+// the global loads 540.  The fp32 MFMA kernel this replaced took 945 us.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -261,6 +274,7 @@ struct GemmTile {
     static constexpr int kLds = 3 * kBuf + 16;
     static constexpr int kFp32A = kSlot * OA::kPitch, kFp32Buf = kFp32A + kSlot * OB::kPitch;
     static_assert(2 * kFp32Buf * 4 <= 3 * kBuf, "the fp32 slots fit the split ones' LDS");
+    static_assert(TN == 2 && (AHEAD == 1 || AHEAD == 2), "a row's two tiles take turns by the slot's parity");
 
     gt_f16 acc[TM][TN];
     OA oa;
@@ -302,6 +316,7 @@ struct GemmTile {
     // the next row, and the slot's splitting and loads, sit among the MFMAs
     // of the row before.  Loads past the last slot repeat it (a branch around
     // a load makes the compiler wait for every load at the join).
+    template <bool LATE>
     __device__ __forceinline__ uint32_t split_slots(int whole, int tail, unsigned tid, volatile int *bad) {
         uint32_t lost = 0;
         Slot in[AHEAD];
@@ -322,7 +337,8 @@ struct GemmTile {
             if (tid == 0) *bad = 0;
         };
         const char *fa = lds + wm0 * 32 + lane * 16, *fb = lds + kABytes + wn0 * 32 + lane * 16;
-        // The products (piece of A, piece of B), the smaller first.
+        // The products (piece of A, piece of B), the smaller first: in a tile
+        // that keeps the first five apart their sum is added before the sixth.
         static constexpr int PA[6] = {2, 1, 1, 0, 0, 0}, PB[6] = {0, 0, 1, 1, 2, 0};
         int cur = 0, nxt = kBuf, wr = 2 * kBuf;  // this slot's buffer, the next one's, the one being written
         gt_bf8 A[2][3], B[TN][3];
@@ -334,18 +350,47 @@ struct GemmTile {
 #pragma unroll
             for (int p = 0; p < 3; p++) B[j][p] = *(const gt_bf8 *)(fb + buf + p * OB::kPlane + j * 1024);
         };
-        // MORE: more slots may follow.  D: the registers holding slot t + 2.
-        const auto slot = [&]<bool MORE, int D>() {
+        // MORE: more slots may follow.  D: the registers holding slot t + 2.  P:
+        // t % 2.  LATE: a row's low sum is added during the next row, behind its
+        // first MFMA (4096^3 593 us, within its own row 617); without it the
+        // stream-K kernel keeps 16 fewer registers live (512x4096x4096 109 us, 115
+        // with it).
+        const auto slot = [&]<bool MORE, int D, int P>() {
+            gt_f16 low;
 #pragma unroll
             for (int i = 0; i < TM; i++) {
                 if (i + 1 < TM) read_a(cur, i + 1, A[(i + 1) & 1]);
                 else if (MORE) read_a(nxt, 0, A[TM & 1]);
-#pragma unroll
-                for (int q = 0; q < 6; q++)
-#pragma unroll
-                    for (int j = 0; j < TN; j++)
+                const auto product = [&](int j, int p) {
+                    if (p < 5 && j == (i + P) % 2)
+                        low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[i & 1][PA[p]], B[j][PB[p]],
+                                                                      p ? low : (gt_f16)(0.f), 0, 0, 0);
+                    else
                         acc[i][j] =
-                            __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[i & 1][PA[q]], B[j][PB[q]], acc[i][j], 0, 0, 0);
+                            __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[i & 1][PA[p]], B[j][PB[p]], acc[i][j], 0, 0, 0);
+                };
+                const int apart = (i + P) % 2, plain = 1 - apart;
+                const auto add_low = [&](int row, int col) {
+#pragma unroll
+                    for (int r = 0; r < 16; r++) acc[row][col][r] += low[r];
+                };
+                if constexpr (LATE) {
+                    product(plain, 0);
+                    if (i > 0) add_low(i - 1, plain);
+                }
+                if (LATE && i < TM - 1) {
+#pragma unroll
+                    for (int p = 0; p < 5; p++) product(plain, p + 1), product(apart, p);
+                } else {
+#pragma unroll
+                    for (int p = 0; p < 5; p++) {
+                        product(apart, p);
+                        if (!LATE || p > 0) product(plain, p);
+                    }
+                    product(plain, 5);
+                    add_low(i, apart);
+                }
+                product(apart, 5);
                 if constexpr (MORE) {
                     if (i == TM - 1) {
 #pragma unroll
@@ -390,7 +435,7 @@ struct GemmTile {
                 put(s0, 0);
                 ready();
                 first();
-                slot.template operator()<false, 0>();
+                slot.template operator()<false, 0, 0>();
                 return lost;
             }
         } else {
@@ -408,19 +453,14 @@ struct GemmTile {
         put(s1, kBuf);
         ready();
         first();
-        // Slot t takes registers t % AHEAD.
-        const auto upto = [&]<int D>(auto &&self, int n) {
-            if constexpr (D < AHEAD) {
-                if (D < n) {
-                    slot.template operator()<true, D>();
-                    self.template operator()<D + 1>(self, n);
-                }
-            }
-        };
+        // Slot t takes registers t % AHEAD and keeps apart by t % 2.
         int t = 0;
 #pragma unroll 1
-        for (; t + AHEAD <= T; t += AHEAD) upto.template operator()<0>(upto, AHEAD);
-        if constexpr (AHEAD > 1) upto.template operator()<0>(upto, T - t);
+        for (; t + 2 <= T; t += 2) {
+            slot.template operator()<true, 0, 0>();
+            slot.template operator()<true, 1 % AHEAD, 1>();
+        }
+        if (t < T) slot.template operator()<true, 0, 0>();
         return lost;
     }
 
@@ -466,6 +506,7 @@ struct GemmTile {
     // ws[row * BN + column], all of it.  tid: threadIdx.x (the stream-K loop
     // passes a copy the compiler cannot see through, so that the lane values
     // are not kept live across tiles).
+    template <bool LATE>
     __device__ __forceinline__ void run(TileCoord tc, int64_t k0, int64_t k1, float *ws, unsigned tid) {
         lane = tid & 63;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -485,7 +526,7 @@ struct GemmTile {
         clear();
         oa.plan(A, args.M - m0, args.lda, tid);
         ob.plan(B, args.N - n0, args.ldb, tid);
-        const uint32_t lost = split_slots(whole, tail, tid, bad);
+        const uint32_t lost = split_slots<LATE>(whole, tail, tid, bad);
         // A non-finite accumulator leaves a non-finite sum of them.
         float sum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
