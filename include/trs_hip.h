@@ -260,7 +260,8 @@ int trs_accumulate_f32(float *dst, const float *src, size_t n);
  * with fewer 256x256 tiles than CUs, at least 90% covered, and a long K
  * (S <= 8, when S slices fill at least half the CUs or give at least as
  * many blocks as the unsplit tile), else one whose 128x128 or 64x128 tile
- * gives at most one block per CU (S <= 16, slices of at least 128 k).  The
+ * gives at most one block per CU (S <= 16, slices of at least 128 k, of 48 where
+ * 64x128 tiles number at most a quarter of the CUs).  The
  * partial products then take S*M*N floats of device memory from the
  * library's block cache for the duration of the call (at most 65,536
  * floats per CU: 64 MiB on a 256-CU device).  If that memory cannot be

@@ -232,9 +232,14 @@ constexpr int64_t kMinSplitDepth = 1024;
 constexpr int64_t kMaxTileSplit = 16;
 constexpr int64_t kMinTileSplitDepth = 128;
 constexpr int64_t kSplitFloatsPerCu = 65536;
-// Time of two 128x128 blocks sharing a CU against one 256x256 block on it,
-// from the measured rates (0.77 and 0.887 of peak): a ragged output takes the
-// large tile when its rounds of blocks, so weighted, are no more.
+// The least k per slice of a few 64x128 tiles (few_tiles in plan_gemm_tiles),
+// and the least K that splits: a split costs its sum's launch, 2.3 us, and a
+// 64x128 tile alone on a CU takes 0.032 us per k.
+constexpr int64_t kMinFewDepth = 48, kMinFewK = 128;
+// Time of two 128x128 blocks sharing a CU against one 256x256 block on it
+// (0.106 and 0.15 us per k with the launch's fixed part, 0.575 without): a
+// ragged output takes the large tile when its rounds of blocks, so weighted,
+// are no more.
 constexpr double kSmallPairOverLarge = 0.575;
 
 // Which kernel a product runs.  Tile choice:
@@ -249,8 +254,18 @@ constexpr double kSmallPairOverLarge = 0.575;
 //     K-slices, when S*tiles reaches half the CUs or at least the block
 //     count of the tile it replaces;
 //   - else 64x128 when 128x128 would give fewer than two blocks per CU and
-//     64x128 divides the shape (76% against 69% of peak measured at
-//     4096x1024x8192), else 128x128 (full or edge-guarded);
+//     64x128 divides the shape (a CU with one block then has two), else
+//     128x128;
+//   - but 64x128 at any shape of 64 rows or more that leaves most CUs without
+//     a block: half a 128x128 block's work on twice the CUs.  A single matrix
+//     of at most a tile per four CUs (beyond, 128x128 in slices is as fast:
+//     700^3 17.5 us, 18.7 on 64x128), split for at most one block per CU in
+//     slices of at least kMinFewDepth; a K below kMinFewK and a batch, which do
+//     not split, while their tiles have a CU each.  128x128 / 64x128, us:
+//     64^3 6.8 / 6.1, 200x400x300 12.2 / 9.1, 300x784x500 13.8 / 11.9,
+//     300x500x100 13.2 / 9.2, 96x6144x96 22.1 / 18.8, 1000x64x1000 7.8 / 7.1,
+//     batches 32 of 100x128x100 9.9 / 8.4, 16 of 300^3 18.3 / 15.2, 8 of
+//     200x200x700 13.9 / 12.0;
 //   - a single matrix whose tile gives at most one block per CU splits K
 //     over that tile (above);
 //   - then stream-K on the 256x256 tile (below) replaces the plan where it
@@ -326,10 +341,14 @@ GemmPlan plan_gemm_tiles(const GemmArgs &g, bool a_plain, bool a_trans, bool b_p
         use_large(large_tiles);
         return p;
     }
-    if (M % 64 == 0 && N % 128 == 0 && K % 32 == 0 && small_tiles < 2 * (int64_t)cu_count) {
+    const int64_t medium_tiles = ceil_div(M, 64) * ceil_div(N, 128) * batch;
+    const bool medium_div = M % 64 == 0 && N % 128 == 0 && K % 32 == 0 && small_tiles < 2 * (int64_t)cu_count;
+    const bool splits = batch == 1 && K >= kMinFewK;
+    const bool few_tiles = !medium_div && M >= 64 && medium_tiles <= (splits ? cu_count / 4 : cu_count);
+    if (medium_div || few_tiles) {
         p.kind = GemmKind::Medium;
         p.bm = 64, p.bn = 128;
-        p.blocks = (M / 64) * (N / 128) * batch;
+        p.blocks = medium_tiles;
     } else {
         p.kind = GemmKind::Small;
         p.bm = 128, p.bn = 128;
@@ -354,9 +373,9 @@ GemmPlan plan_gemm_tiles(const GemmArgs &g, bool a_plain, bool a_trans, bool b_p
             return p;
         }
     }
-    if (batch == 1 && p.blocks <= cu_count) {
-        int64_t S = std::min<int64_t>(kMaxTileSplit, 2 * (int64_t)cu_count / p.blocks);
-        S = std::min<int64_t>(S, K / kMinTileSplitDepth);
+    if (batch == 1 && p.blocks <= cu_count && (splits || !few_tiles)) {
+        int64_t S = std::min<int64_t>(kMaxTileSplit, (few_tiles ? 1 : 2) * (int64_t)cu_count / p.blocks);
+        S = std::min<int64_t>(S, K / (few_tiles ? kMinFewDepth : kMinTileSplitDepth));
         S = std::min<int64_t>(S, kSplitFloatsPerCu * cu_count / (M * N));
         if (S >= 2) {
             const int64_t ks = ((K + S - 1) / S + p.bk - 1) / p.bk * p.bk;
@@ -374,20 +393,23 @@ GemmPlan plan_gemm_tiles(const GemmArgs &g, bool a_plain, bool a_trans, bool b_p
     return p;
 }
 
-// Stream-K on the LDS-loading 256x256 tile: one block per CU, each taking
+// Stream-K on the 256x256 tile: one block per CU, each taking
 // an equal share of the product's (tile, slice) units, then one pass adding
-// the pieces of the tiles split between blocks (gemm_f32_mfma_lds_sk).  It
+// the pieces of the tiles split between blocks (gemm_split_tile_sk).  It
 // removes the idle CUs of a last, partial round of tiles (6144^3: 576
 // tiles, three rounds of 256 for 2.25 rounds of work) and of outputs with
 // fewer tiles than CUs that no power-of-two K split fills (3072^3: 144).
 //
 // The choice compares estimated times in k steps of one 256x256 tile on one
-// CU (0.21 us at the measured 0.92 of peak): the plan above by its rounds of
+// CU (0.15 us at 4096^3): the plan above by its rounds of
 // blocks, and stream-K by its even share plus kStreamKCost for the pieces'
 // extra traffic (two 256 KiB pieces per split tile written, read back and
 // added, at most one split tile per block), the fix-up launch and a block's
 // extra segment starts.  The 128x128 and 64x128 tiles cost 0.30 and 0.175
-// of a large k step per k (their measured rates and areas).  Stream-K needs
+// of a large k step per k (their rates and areas; alone on a CU a 64x128 block
+// takes 0.032 us per k, 0.21 of one).  Against every tile and split of 30
+// shapes the choice is the fastest or within a few percent, at most 12% off
+// (512x4096x4096 113 us, 101 in 8 large slices; 2048^3 109 and 101).  Stream-K needs
 // tiles at least 85% covered, no K split of its own (ktotal), and at least
 // kStreamKMinWork k steps per CU.
 constexpr double kStreamKCost = 150.0;
