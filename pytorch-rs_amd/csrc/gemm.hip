@@ -236,10 +236,10 @@ constexpr int64_t kSplitFloatsPerCu = 65536;
 // and the least K that splits: a split costs its sum's launch, 2.3 us, and a
 // 64x128 tile alone on a CU takes 0.032 us per k.
 constexpr int64_t kMinFewDepth = 48, kMinFewK = 128;
-// Time of two 128x128 blocks sharing a CU against one 256x256 block on it
-// (0.106 and 0.15 us per k with the launch's fixed part, 0.575 without): a
-// ragged output takes the large tile when its rounds of blocks, so weighted,
-// are no more.
+// Time of two 128x128 blocks sharing a CU against one 256x256 block on it,
+// from the FP32 MFMA tiles' rates; these run 0.106 us per k at 32 x 512^3,
+// its fixed part included, against 0.15 at 4096^3.  A ragged output takes the
+// large tile when its rounds of blocks, so weighted, are no more.
 constexpr double kSmallPairOverLarge = 0.575;
 
 // Which kernel a product runs.  Tile choice:

@@ -1,5 +1,5 @@
 // lds_dma.h -- loading global memory straight into LDS
-// (global_load_lds_dwordx4), shared by the GEMM and skinny-product kernels.
+// (global_load_lds_dwordx4), used by the skinny-product kernels.
 #pragma once
 
 #include <hip/hip_runtime.h>
