@@ -6,21 +6,21 @@
 // fp32 inputs and fp32 accumulation ("highest" precision,
 // python/torch_rs/__init__.py:81-85) but sums in MFMA order, so it is checked
 // against the reference within |dC| <= 1e-5*sqrt(K)*(|A||B|).  The products
-// run on the bf16 matrix cores, each float as three bf16 pieces, with a
-// smaller error than the fp32 MFMA's (gemm_tile.h).
+// run on the bf16 matrix cores, each float as three bf16 pieces (gemm_tile.h
+// has the error, which is that of fp32 MFMA or less).
 //
 // Three tiles (GemmTile), each in the four operand layouts and at any M, N
 // and K (rows past the edge repeat the last one and are not stored):
-//   256x256  8 waves of 128x64, one block per CU (144 KB of LDS)
-//   128x128  4 waves of 64x64, or where blocks do not fill the CUs twice 8 of
-//            32x64; two blocks per CU
+//   256x256  two 256x128 halves one after the other, 8 waves of 64x64, one
+//            block per CU (108 KB of LDS)
+//   128x128  4 waves of 64x64, two blocks per CU, or where blocks do not fill
+//            the CUs twice 8 of 32x64, one per CU
 //   64x128   4 waves of 32x64, two blocks per CU
 // The 4-wave 128x128 tile reads a third less from LDS per product, which
 // counts where the whole chip runs it and power sets the clock (batched
 // 32x512^3 52.3 us against 54.0, 1000x2047x1500 48.4 against 50.3); the 8-wave
 // one issues its slot in half the instructions per wave, which counts where
-// one block has a CU to itself (200x300x400 12.4 us against 14.6, 700^3 16.6
-// against 18.8, 64^3 6.6 against 8.1).
+// one block has a CU to itself (700^3 16.6 us against 18.8).
 // Blocks are remapped so that consecutive tiles share an XCD (each XCD has
 // its own L2), and tiles are walked in groups of kGroupM tile rows.
 #include <hip/hip_runtime.h>
@@ -36,9 +36,9 @@ namespace trs {
 namespace {
 
 template <bool AKC, bool BKC>
-using LargeTile = GemmTile<256, 256, 2, 4, 1, AKC, BKC>;
+using LargeTile = GemmTile<256, 128, 4, 2, 1, AKC, BKC, 2>;
 template <bool AKC, bool BKC>
-using SmallTile = GemmTile<128, 128, 2, 2, 2, AKC, BKC>;
+using SmallTile = GemmTile<128, 128, 2, 2, 1, AKC, BKC>;
 template <bool AKC, bool BKC>
 using SmallTile8 = GemmTile<128, 128, 4, 2, 1, AKC, BKC>;
 template <bool AKC, bool BKC>
@@ -56,15 +56,16 @@ inline int slice_depth(const GemmArgs &g, bool a_plain) {
 
 // One block per tile.
 template <class T, int MINB>
-__global__ void __launch_bounds__(T::NT, MINB) gemm_split_tile(GemmArgs args) {
+__global__ void __launch_bounds__(T::NT, MINB) gemm_split_tile(GemmArgs) {
+    GemmArgsRef args = kernel_args();
     __shared__ __attribute__((aligned(1024))) char lds[T::kLds];
     uint32_t bid = blockIdx.x;
     if (args.xcd_remap) {
         const uint32_t per_xcd = gridDim.x / kXcds;
         bid = (bid % kXcds) * per_xcd + bid / kXcds;
     }
-    T tile(args, lds);
-    tile.template run<true>(decode_tile(args, bid), 0, INT64_MAX, nullptr, threadIdx.x);
+    T tile((gt_lds)lds);
+    tile.run(args, decode_tile(args, bid), 0, INT64_MAX, nullptr);
 }
 
 // Stream-K: one persistent block per CU, block b taking the (tile, slice)
@@ -76,20 +77,20 @@ __global__ void __launch_bounds__(T::NT, MINB) gemm_split_tile(GemmArgs args) {
 // for another.  Logical block b runs as blockIdx (b % (G/8)) * 8 + b / (G/8),
 // so each XCD takes one contiguous eighth of the units.
 template <class T>
-__global__ void __launch_bounds__(T::NT, 1) gemm_split_tile_sk(GemmArgs args) {
+__global__ void __launch_bounds__(T::NT, 1) gemm_split_tile_sk(GemmArgs) {
+    GemmArgsRef first = kernel_args();
     __shared__ __attribute__((aligned(1024))) char lds[T::kLds];
-    const int64_t G = args.sk_blocks, U = args.sk_units, Q = args.sk_q;
-    const int64_t b = args.xcd_remap ? (blockIdx.x % kXcds) * (G / kXcds) + blockIdx.x / kXcds : blockIdx.x;
+    const int64_t G = first.sk_blocks, U = first.sk_units, Q = first.sk_q;
+    const int64_t b = first.xcd_remap ? (blockIdx.x % kXcds) * (G / kXcds) + blockIdx.x / kXcds : blockIdx.x;
     const int64_t u0 = b * U / G, u1 = (b + 1) * U / G;
     // Segment: slices [qb, qe) of tile t; the next starts the next tile.
     int64_t t = u0 / Q, qb = u0 - t * Q;
     for (int64_t u = u0; u < u1; t++, qb = 0) {
+        GemmArgsRef args = kernel_args();
         const int64_t qe = imin(Q, qb + (u1 - u));
         float *ws = (qb == 0 && qe == Q) ? nullptr : args.sk_ws + (2 * b + (u == u0 ? 0 : 1)) * kLargeTileFloats;
-        unsigned tid = threadIdx.x;
-        asm volatile("" : "+v"(tid));
-        T tile(args, lds);
-        tile.template run<false>(decode_tile(args, (uint32_t)t), qb * args.sk_depth, qe * args.sk_depth, ws, tid);
+        T tile((gt_lds)lds);
+        tile.run(args, decode_tile(args, (uint32_t)t), qb * args.sk_depth, qe * args.sk_depth, ws);
         u += qe - qb;
     }
 }
@@ -97,7 +98,8 @@ __global__ void __launch_bounds__(T::NT, 1) gemm_split_tile_sk(GemmArgs args) {
 // The pieces of the tiles stream-K split between blocks, added in k order
 // (block order) into C.  Block (t, y) takes rows 16y..16y+15 of tile t; a
 // tile that one block ran whole was stored by it and is skipped.
-__global__ void __launch_bounds__(256) gemm_streamk_fixup(GemmArgs args) {
+__global__ void __launch_bounds__(256) gemm_streamk_fixup(GemmArgs) {
+    GemmArgsRef args = kernel_args();
     const int64_t G = args.sk_blocks, U = args.sk_units, Q = args.sk_q;
     const int64_t t = blockIdx.x;
     // The block whose units hold unit u: the largest b with b*U/G <= u.
@@ -294,7 +296,7 @@ int launch_kind(GemmKind kind, const GemmArgs &g, bool a_plain, bool b_plain, in
         case GemmKind::Large: return launch_tile<LargeTile<AKC, BKC>, 1>(g, kLarge, kLarge, s);
         case GemmKind::Medium: return launch_tile<MediumTile<AKC, BKC>, 2>(g, 64, 128, s);
         default:
-            if (alone) return launch_tile<SmallTile8<AKC, BKC>, 2>(g, 128, 128, s);
+            if (alone) return launch_tile<SmallTile8<AKC, BKC>, 1>(g, 128, 128, s);
             return launch_tile<SmallTile<AKC, BKC>, 2>(g, 128, 128, s);
         }
     });

@@ -5,29 +5,43 @@
 // h = rn(x), m = rn(x - h), l = x - h - m (bf16 has 8 significant bits and
 // float's exponent range, so nothing is scaled).  Of the nine products of
 // two such sums the six of weight 2^-16 and above are computed, each exact in
-// the matrix cores and added in fp32, the small ones first; the three left
-// out are below 2^-24 of |x||y| together.  bf16 MFMA runs 16 times the rate of
+// the matrix cores and added in fp32.  bf16 MFMA runs 16 times the rate of
 // fp32 MFMA, so six products cost 3/8 of the fp32 instruction's time.
 // Rounding to nearest matters: with truncated pieces every small product has
 // the sign of the whole one, and the accumulator's alignment loses them in
 // one direction (K = 4096 on positive data: 9.5e-6).
 //
-// The matrix core rounds the accumulator once per 8 k, so six products of 16 k
-// round it 12 times where fp32 MFMA does 8.  So each MFMA tile takes the five
-// small products of every other slot in a sum of their own (`low`) and adds
-// that once: 3 roundings there, 7.5 on average.  Half the MFMA tiles do it in
-// one slot and the other half in the next, which spreads the adds.  In every
-// slot for every tile it halves the error again, at 634 us for 4096^3; not at
-// all, operands with many zeros (a relu's output), which fp32 MFMA adds without
-// rounding, have up to 1.2 times its error (565 us); this way 593 us.
+// Two sums are kept over all of K: `acc` of the leading products h h, and
+// `low` of the five small ones, added to it once at the end.  `low` is 2^-8 of
+// the result and its roundings do not count; `acc` adds products of 16 bits,
+// rounded once per 8 k by the matrix core and mostly exactly.  An fp32 MFMA
+// rounds a nonzero product each.  Adding `low` once per slot instead gives
+// back a rounding a slot, which operands with many zeros (a relu's output
+// under dropout, one-hot rows) show: with a 0.02 share of nonzeros it is
+// behind fp32 MFMA (1.1 times its error), and with the small products added
+// straight to `acc` in half the slots, which was faster (583 us at 4096^3),
+// from a share of 0.35 down (1.6 times at 0.02).  The price is registers: a
+// 256x256 tile has room for one sum only, so it is computed as two halves of
+// 256x128, each splitting A again.
 //
-// Error against 64 bits (2-norm over sqrt of the sum of squares; the fp32 MFMA
-// tiles this replaced on the same inputs in brackets), [1000, K] @ [K, 1000]
-// of relu(N(0,1)) and U(-1, 1)/sqrt(K): K = 64 8.6e-8 (1.05e-7), K = 512
-// 1.30e-7 (1.50e-7), K = 2048 1.86e-7 (2.1e-7), K = 6144 2.31e-7 (2.58e-7),
-// K = 16384 3.8e-7 (4.1e-7); N(0,1) and |N(0,1)| are further below.  Of the
-// training step [2048,1024] -> 1500 -> 512: out 3.1e-7, dX 2.5e-7, dW1
-// 2.2e-7, dW2 5.9e-8 (6.9e-8 to 7.2e-8).
+// Error against 64 bits (2-norm over 2-norm; the fp32 MFMA tiles this replaced
+// on the same inputs in brackets), [1000, K] @ [K, 1000], normal values, left
+// operand with the given share of nonzeros:
+//   K       1                  0.25               0.05               0.005
+//     64    5.0e-8 (1.4e-7)    3.4e-8 (7.6e-8)    2.7e-8 (4.0e-8)    2.6e-8 (2.8e-8)
+//    512    7.7e-8 (2.1e-7)    5.9e-8 (1.1e-7)    5.0e-8 (6.6e-8)    3.9e-8 (4.1e-8)
+//   6144    1.3e-7 (3.6e-7)    1.0e-7 (1.9e-7)    8.5e-8 (1.1e-7)    7.6e-8 (8.0e-8)
+// and 4096^3 4.0e-7 (1.15e-6), 2.3e-7 (5.7e-7), 9.7e-8 (2.6e-7), 3.8e-8 (8.5e-8).
+// The one case behind is an output, or a K slice's part of it, that is a single
+// nonzero product: the three products left out, below 2^-24 of it together,
+// take a diagonal operand from 2.52e-8 to 2.59e-8 (4% of such outputs are the
+// neighbour of the correctly rounded product) and [64, 512] @ [512, 200] in 8
+// slices with a 0.02 share of nonzeros from 5.52e-8 to 5.58e-8.
+//
+// An output of a tile depends on its row of A and its column of B alone,
+// wherever they stand in it.  The order of the products is not symmetric in A
+// and B, so A @ A.mT is symmetric to rounding only; and a tile that falls back
+// to fp32 MFMA (below) rounds all its outputs as that does.
 //
 // Where the split does not hold -- a value whose lowest bits fall below
 // bf16's smallest subnormal (|x| < 2^-110 with low bits set), an infinity, a
@@ -35,11 +49,9 @@
 // MFMA (fp32_slots): the split notes lost bits as it goes, and everything
 // else leaves a non-finite accumulator.
 //
-// What bounds it: the card's power.  At 4096^3 random values run 593 us
-// (1,390 TFLOP/s of bf16).  With every product added straight to the
-// accumulator a product of zeros ran 416 us (1,980 TFLOP/s) and random values
-// 570 us at a lower clock: the MFMAs alone 466 us, with their LDS reads 490, with
-// the global loads 540.  The fp32 MFMA kernel this replaced took 945 us.
+// What bounds it: the card's power.  At 4096^3 random values run 640-670 us
+// (1,230-1,290 TFLOP/s of bf16), zeros in far less at a higher clock.  The fp32
+// MFMA kernel this replaced took 950 us.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -54,6 +66,9 @@ typedef float gt_f16 __attribute__((ext_vector_type(16)));
 typedef uint32_t gt_u4 __attribute__((ext_vector_type(4)));
 typedef const float __attribute__((address_space(1))) *gt_global;
 typedef const char __attribute__((address_space(1))) *gt_global_bytes;
+typedef char __attribute__((address_space(3))) *gt_lds;
+typedef float __attribute__((address_space(3))) *gt_lds_floats;
+typedef volatile int __attribute__((address_space(3))) *gt_flag;
 typedef __bf16 gt_bf2 __attribute__((ext_vector_type(2)));
 typedef __bf16 gt_bf8 __attribute__((ext_vector_type(8)));
 
@@ -79,6 +94,16 @@ struct GemmArgs {
     float *sk_ws;
 };
 
+// The kernel's arguments, read where they are used: from a copy of the pointer
+// to them that the compiler cannot see through, so that a loop's fields are
+// loaded again on each turn and not held in scalar registers over all of it.
+typedef const GemmArgs __attribute__((address_space(4))) &GemmArgsRef;
+__device__ __forceinline__ GemmArgsRef kernel_args() {
+    auto p = (const GemmArgs __attribute__((address_space(4))) *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *p;
+}
+
 constexpr int kGroupM = 8;
 constexpr int kXcds = 8;
 constexpr int kSlot = 16;  // k per slot: the depth of one v_mfma_f32_32x32x16_bf16
@@ -103,7 +128,7 @@ struct TileCoord {
 // kGroupM tile rows, the group's tiles taken down its columns.  In 32 bits: a
 // grid has below 2^31 tiles, and the 64-bit divisions are software loops of
 // some 600 instructions before a block's first load.
-__device__ __forceinline__ TileCoord decode_tile(const GemmArgs &args, uint32_t t) {
+__device__ __forceinline__ TileCoord decode_tile(GemmArgsRef args, uint32_t t) {
     const uint32_t tm = (uint32_t)args.tiles_m, tn = (uint32_t)args.tiles_n, tiles = tm * tn;
     TileCoord c;
     const uint32_t batch = t / tiles;
@@ -235,8 +260,9 @@ struct SlotOperand {
             }
         }
     }
-    __device__ __forceinline__ void store_split(const Regs &v, char *lds, uint32_t &lost) const {
+    __device__ __forceinline__ void store_split(const Regs &v, gt_lds lds, uint32_t &lost) const {
         typedef uint32_t Pack __attribute__((ext_vector_type(CH / 2)));
+        typedef Pack __attribute__((address_space(3))) *PackLds;
 #pragma unroll
         for (int q = 0; q < NC; q++) {
             Pack h, m, l;
@@ -246,14 +272,14 @@ struct SlotOperand {
                 split_pair(v[q][2 * e], v[q][2 * e + 1], x, y, z, lost);
                 h[e] = x, m[e] = y, l[e] = z;
             }
-            char *d = lds + (row[q] >> 5) * 1024 + (k[q] >> 3) * 512 + (row[q] & 31) * 16 + (k[q] & 7) * 2;
-            *(Pack *)d = h;
-            *(Pack *)(d + kPlane) = m;
-            *(Pack *)(d + 2 * kPlane) = l;
+            const gt_lds d = lds + (row[q] >> 5) * 1024 + (k[q] >> 3) * 512 + (row[q] & 31) * 16 + (k[q] & 7) * 2;
+            *(PackLds)d = h;
+            *(PackLds)(d + kPlane) = m;
+            *(PackLds)(d + 2 * kPlane) = l;
         }
     }
     // As floats, [k][row]: the pitch puts k and k + 1 half the banks apart.
-    __device__ __forceinline__ void store_fp32(const Regs &v, float *lds) const {
+    __device__ __forceinline__ void store_fp32(const Regs &v, gt_lds_floats lds) const {
 #pragma unroll
         for (int q = 0; q < NC; q++)
 #pragma unroll
@@ -264,7 +290,7 @@ struct SlotOperand {
 // A BM x BN tile of C on WGM x WGN waves, each (BM/WGM) x (BN/WGN) as 32x32
 // MFMA tiles.  AHEAD slots are on their way from memory in registers (the
 // depth is not what bounds it: 1, 2 and 3 measured within 1%).  AKC, BKC: the operand is contiguous along k.
-template <int BM, int BN, int WGM, int WGN, int AHEAD, bool AKC, bool BKC>
+template <int BM, int BN, int WGM, int WGN, int AHEAD, bool AKC, bool BKC, int PARTS = 1>
 struct GemmTile {
     static constexpr int NT = WGM * WGN * 64, WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
     using OA = SlotOperand<BM, NT, AKC>;
@@ -274,17 +300,18 @@ struct GemmTile {
     static constexpr int kLds = 3 * kBuf + 16;
     static constexpr int kFp32A = kSlot * OA::kPitch, kFp32Buf = kFp32A + kSlot * OB::kPitch;
     static_assert(2 * kFp32Buf * 4 <= 3 * kBuf, "the fp32 slots fit the split ones' LDS");
-    static_assert(TN == 2 && (AHEAD == 1 || AHEAD == 2), "a row's two tiles take turns by the slot's parity");
+    static_assert(AHEAD == 1 || AHEAD == 2, "the slot loop is unrolled over two register sets");
 
-    gt_f16 acc[TM][TN];
+    // The products of the leading pieces, and all the others'.
+    gt_f16 acc[TM][TN], low[TM][TN];
     OA oa;
     OB ob;
-    char *lds;
-    const GemmArgs &args;
+    gt_lds lds;
+    int64_t lda, ldb;
     int64_t astep, bstep;
     int lane, wm0, wn0;
 
-    __device__ __forceinline__ GemmTile(const GemmArgs &a, char *l) : lds(l), args(a) {}
+    __device__ __forceinline__ explicit GemmTile(gt_lds l) : lds(l) {}
 
     __device__ __forceinline__ void clear() {
 #pragma unroll
@@ -292,15 +319,15 @@ struct GemmTile {
 #pragma unroll
             for (int j = 0; j < TN; j++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+                for (int r = 0; r < 16; r++) acc[i][j][r] = low[i][j][r] = 0.f;
     }
     struct Slot {  // a slot's floats on their way to LDS
         typename OA::Regs a;
         typename OB::Regs b;
     };
     __device__ __forceinline__ void load(Slot &r) const {
-        oa.load(r.a, args.lda);
-        ob.load(r.b, args.ldb);
+        oa.load(r.a, lda);
+        ob.load(r.b, ldb);
     }
 
     // `whole` slots from the operands' current pointers on, after the `tail`
@@ -316,8 +343,7 @@ struct GemmTile {
     // the next row, and the slot's splitting and loads, sit among the MFMAs
     // of the row before.  Loads past the last slot repeat it (a branch around
     // a load makes the compiler wait for every load at the join).
-    template <bool LATE>
-    __device__ __forceinline__ uint32_t split_slots(int whole, int tail, unsigned tid, volatile int *bad) {
+    __device__ __forceinline__ uint32_t split_slots(int whole, int tail, unsigned tid, gt_flag bad) {
         uint32_t lost = 0;
         Slot in[AHEAD];
         const int T = whole + (tail ? 1 : 0);
@@ -336,7 +362,8 @@ struct GemmTile {
             __syncthreads();
             if (tid == 0) *bad = 0;
         };
-        const char *fa = lds + wm0 * 32 + lane * 16, *fb = lds + kABytes + wn0 * 32 + lane * 16;
+        typedef const gt_bf8 __attribute__((address_space(3))) *Frag;
+        const gt_lds fa = lds + wm0 * 32 + lane * 16, fb = lds + kABytes + wn0 * 32 + lane * 16;
         // The products (piece of A, piece of B), the smaller first: in a tile
         // that keeps the first five apart their sum is added before the sixth.
         static constexpr int PA[6] = {2, 1, 1, 0, 0, 0}, PB[6] = {0, 0, 1, 1, 2, 0};
@@ -344,53 +371,25 @@ struct GemmTile {
         gt_bf8 A[2][3], B[TN][3];
         const auto read_a = [&](int buf, int i, gt_bf8 (&d)[3]) {
 #pragma unroll
-            for (int p = 0; p < 3; p++) d[p] = *(const gt_bf8 *)(fa + buf + p * OA::kPlane + i * 1024);
+            for (int p = 0; p < 3; p++) d[p] = *(Frag)(fa + buf + p * OA::kPlane + i * 1024);
         };
         const auto read_b = [&](int buf, int j) {
 #pragma unroll
-            for (int p = 0; p < 3; p++) B[j][p] = *(const gt_bf8 *)(fb + buf + p * OB::kPlane + j * 1024);
+            for (int p = 0; p < 3; p++) B[j][p] = *(Frag)(fb + buf + p * OB::kPlane + j * 1024);
         };
-        // MORE: more slots may follow.  D: the registers holding slot t + 2.  P:
-        // t % 2.  LATE: a row's low sum is added during the next row, behind its
-        // first MFMA (4096^3 593 us, within its own row 617); without it the
-        // stream-K kernel keeps 16 fewer registers live (512x4096x4096 109 us, 115
-        // with it).
-        const auto slot = [&]<bool MORE, int D, int P>() {
-            gt_f16 low;
+        // MORE: more slots may follow.  D: the registers holding slot t + 2.
+        const auto slot = [&]<bool MORE, int D>() {
 #pragma unroll
             for (int i = 0; i < TM; i++) {
                 if (i + 1 < TM) read_a(cur, i + 1, A[(i + 1) & 1]);
                 else if (MORE) read_a(nxt, 0, A[TM & 1]);
-                const auto product = [&](int j, int p) {
-                    if (p < 5 && j == (i + P) % 2)
-                        low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[i & 1][PA[p]], B[j][PB[p]],
-                                                                      p ? low : (gt_f16)(0.f), 0, 0, 0);
-                    else
-                        acc[i][j] =
-                            __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[i & 1][PA[p]], B[j][PB[p]], acc[i][j], 0, 0, 0);
-                };
-                const int apart = (i + P) % 2, plain = 1 - apart;
-                const auto add_low = [&](int row, int col) {
 #pragma unroll
-                    for (int r = 0; r < 16; r++) acc[row][col][r] += low[r];
-                };
-                if constexpr (LATE) {
-                    product(plain, 0);
-                    if (i > 0) add_low(i - 1, plain);
-                }
-                if (LATE && i < TM - 1) {
+                for (int p = 0; p < 6; p++)
 #pragma unroll
-                    for (int p = 0; p < 5; p++) product(plain, p + 1), product(apart, p);
-                } else {
-#pragma unroll
-                    for (int p = 0; p < 5; p++) {
-                        product(apart, p);
-                        if (!LATE || p > 0) product(plain, p);
+                    for (int j = 0; j < TN; j++) {
+                        gt_f16 &d = p < 5 ? low[i][j] : acc[i][j];
+                        d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[i & 1][PA[p]], B[j][PB[p]], d, 0, 0, 0);
                     }
-                    product(plain, 5);
-                    add_low(i, apart);
-                }
-                product(apart, 5);
                 if constexpr (MORE) {
                     if (i == TM - 1) {
 #pragma unroll
@@ -398,11 +397,11 @@ struct GemmTile {
                     }
                     if (i == 0) oa.store_split(in[D].a, lds + wr, lost);
                     if (i == (TM > 1 ? 1 : 0)) {
-                        oa.load(in[D].a, args.lda);
+                        oa.load(in[D].a, lda);
                         ob.store_split(in[D].b, lds + wr + kABytes, lost);
                     }
                     if (i == (TM > 2 ? 2 : TM - 1)) {
-                        ob.load(in[D].b, args.ldb);
+                        ob.load(in[D].b, ldb);
                         move_on();
                     }
                 }
@@ -429,13 +428,13 @@ struct GemmTile {
             OB tb = ob;
             ta.advance(whole * astep);
             tb.advance(whole * bstep);
-            ta.load_tail(s0.a, args.lda, tail);
-            tb.load_tail(s0.b, args.ldb, tail);
+            ta.load_tail(s0.a, lda, tail);
+            tb.load_tail(s0.b, ldb, tail);
             if (!whole) {
                 put(s0, 0);
                 ready();
                 first();
-                slot.template operator()<false, 0, 0>();
+                slot.template operator()<false, 0>();
                 return lost;
             }
         } else {
@@ -453,37 +452,37 @@ struct GemmTile {
         put(s1, kBuf);
         ready();
         first();
-        // Slot t takes registers t % AHEAD and keeps apart by t % 2.
+        // Slot t takes registers t % AHEAD.
         int t = 0;
 #pragma unroll 1
         for (; t + 2 <= T; t += 2) {
-            slot.template operator()<true, 0, 0>();
-            slot.template operator()<true, 1 % AHEAD, 1>();
+            slot.template operator()<true, 0>();
+            slot.template operator()<true, 1 % AHEAD>();
         }
-        if (t < T) slot.template operator()<true, 0, 0>();
+        if (t < T) slot.template operator()<true, 0>();
         return lost;
     }
 
     // The same slots on fp32 MFMA (v_mfma_f32_32x32x2_f32), double-buffered.
     __device__ __forceinline__ void fp32_slots(int whole, int tail) {
         Slot in;
-        float *f = (float *)lds;
+        const gt_lds_floats f = (gt_lds_floats)lds;
         const int T = whole + (tail ? 1 : 0);
         const auto fetch = [&](int t) {
             if (t < whole) load(in);
-            else oa.load_tail(in.a, args.lda, tail), ob.load_tail(in.b, args.ldb, tail);
+            else oa.load_tail(in.a, lda, tail), ob.load_tail(in.b, ldb, tail);
             oa.advance(astep);
             ob.advance(bstep);
         };
         fetch(0);
         for (int t = 0; t < T; t++) {
-            float *buf = f + (t & 1) * kFp32Buf;
+            const gt_lds_floats buf = f + (t & 1) * kFp32Buf;
             oa.store_fp32(in.a, buf);
             ob.store_fp32(in.b, buf + kFp32A);
             if (t + 1 < T) fetch(t + 1);
             __syncthreads();
-            const float *pa = buf + (lane >> 5) * OA::kPitch + wm0 + (lane & 31);
-            const float *pb = buf + kFp32A + (lane >> 5) * OB::kPitch + wn0 + (lane & 31);
+            const gt_lds_floats pa = buf + (lane >> 5) * OA::kPitch + wm0 + (lane & 31);
+            const gt_lds_floats pb = buf + kFp32A + (lane >> 5) * OB::kPitch + wn0 + (lane & 31);
 #pragma unroll 2
             for (int k = 0; k < kSlot; k += 2) {
                 float x[TM], y[TN];
@@ -501,32 +500,51 @@ struct GemmTile {
         __syncthreads();
     }
 
-    // The tile over its k in [k0, k1) (k1 past the last k: to the end; k0 a
-    // multiple of 16).  Stores it into C, or with `ws` set into
-    // ws[row * BN + column], all of it.  tid: threadIdx.x (the stream-K loop
-    // passes a copy the compiler cannot see through, so that the lane values
-    // are not kept live across tiles).
-    template <bool LATE>
-    __device__ __forceinline__ void run(TileCoord tc, int64_t k0, int64_t k1, float *ws, unsigned tid) {
+    // The block's tile over its k in [k0, k1) (k1 past the last k: to the end;
+    // k0 a multiple of 16): PARTS times BN columns, one after the other.
+    // Stores it into C, or with `ws` set into ws[row * PARTS * BN + column].
+    __device__ __forceinline__ void run(GemmArgsRef args, TileCoord tc, int64_t k0, int64_t k1, float *ws) {
+        if constexpr (PARTS == 1) {
+            run_part(args, tc.batch, tc.m * BM, tc.n * BN, k0, k1, ws, threadIdx.x);
+        } else {
+#pragma unroll 1
+            for (int part = 0; part < PARTS; part++) {
+                GemmArgsRef again = kernel_args();
+                const int64_t n0 = (tc.n * PARTS + part) * BN;
+                if (part && n0 >= again.N) break;
+                // Nor is what a lane derives from its number kept over the parts.
+                unsigned tid = threadIdx.x;
+                asm volatile("" : "+v"(tid));
+                run_part(again, tc.batch, tc.m * BM, n0, k0, k1, ws ? ws + part * BN : nullptr, tid);
+            }
+        }
+    }
+
+    __device__ __forceinline__ void run_part(GemmArgsRef args, int64_t batch, int64_t m0, int64_t n0, int64_t k0,
+                                             int64_t k1, float *ws, unsigned tid) {
+        lda = args.lda, ldb = args.ldb;
         lane = tid & 63;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         wm0 = (wave / WGN) * WM;
         wn0 = (wave % WGN) * WN;
-        const int64_t Kb = args.ktotal ? imin(args.K, args.ktotal - tc.batch * args.K) : args.K;
-        const int64_t m0 = tc.m * BM, n0 = tc.n * BN;
-        const float *A = args.a + tc.batch * args.bsa + (AKC ? m0 * args.lda + k0 : m0 + k0 * args.lda);
-        const float *B = args.b + tc.batch * args.bsb + (BKC ? n0 * args.ldb + k0 : n0 + k0 * args.ldb);
-        astep = AKC ? kSlot : kSlot * args.lda;
-        bstep = BKC ? kSlot : kSlot * args.ldb;
+        const int64_t Kb = args.ktotal ? imin(args.K, args.ktotal - batch * args.K) : args.K;
+        const float *A = args.a + batch * args.bsa + (AKC ? m0 * lda + k0 : m0 + k0 * lda);
+        const float *B = args.b + batch * args.bsb + (BKC ? n0 * ldb + k0 : n0 + k0 * ldb);
+        astep = AKC ? kSlot : kSlot * lda;
+        bstep = BKC ? kSlot : kSlot * ldb;
         const int64_t kspan = imin(k1, Kb) - k0;
         // 64-bit compares run on the vector units; back to scalar registers.
         const int whole = __builtin_amdgcn_readfirstlane((int)(kspan >> 4));
         const int tail = __builtin_amdgcn_readfirstlane((int)(kspan & (kSlot - 1)));
-        volatile int *bad = (volatile int *)(lds + 3 * kBuf);
+        const gt_flag bad = (gt_flag)(lds + 3 * kBuf);
         clear();
-        oa.plan(A, args.M - m0, args.lda, tid);
-        ob.plan(B, args.N - n0, args.ldb, tid);
-        const uint32_t lost = split_slots<LATE>(whole, tail, tid, bad);
+        oa.plan(A, args.M - m0, lda, tid);
+        ob.plan(B, args.N - n0, ldb, tid);
+        const uint32_t lost = split_slots(whole, tail, tid, bad);
+        // What follows works its lane values out again, so that the slot loop
+        // does not keep them live.
+        asm volatile("" : "+v"(tid));
+        lane = tid & 63;
         // A non-finite accumulator leaves a non-finite sum of them.
         float sum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -534,16 +552,20 @@ struct GemmTile {
 #pragma unroll
             for (int j = 0; j < TN; j++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) sum[r & 3] += acc[i][j][r];
+                for (int r = 0; r < 16; r++) {
+                    acc[i][j][r] += low[i][j][r];
+                    sum[r & 3] += acc[i][j][r];
+                }
         const float s = (sum[0] + sum[1]) + (sum[2] + sum[3]);
         if ((lost & 0xffffu) != 0 || !(__builtin_fabsf(s) < __builtin_inff())) *bad = 1;
         __syncthreads();
         if (__builtin_expect(__builtin_amdgcn_readfirstlane(*bad), 0)) {
             clear();
-            oa.plan(A, args.M - m0, args.lda, tid);
-            ob.plan(B, args.N - n0, args.ldb, tid);
+            oa.plan(A, args.M - m0, lda, tid);
+            ob.plan(B, args.N - n0, ldb, tid);
             fp32_slots(whole, tail);
         }
+        GemmArgsRef out = PARTS == 1 ? args : kernel_args();
         // Lane l, register r of a 32x32 tile: row 8*(r/4) + 4*(l/32) + r%4, column l%32.
         const int rl = 4 * (lane >> 5), cl = lane & 31;
         if (ws) {
@@ -553,18 +575,18 @@ struct GemmTile {
                 for (int j = 0; j < TN; j++)
 #pragma unroll
                     for (int r = 0; r < 16; r++)
-                        ws[(wm0 + i * 32 + 8 * (r / 4) + rl + r % 4) * BN + wn0 + j * 32 + cl] = acc[i][j][r];
+                        ws[(wm0 + i * 32 + 8 * (r / 4) + rl + r % 4) * (PARTS * BN) + wn0 + j * 32 + cl] = acc[i][j][r];
             return;
         }
-        float *C = args.c + tc.batch * args.bsc;
+        float *C = out.c + batch * out.bsc;
         const int64_t mrow = m0 + wm0 + rl, ncol = n0 + wn0 + cl;
-        float *cp = C + mrow * args.ldc + ncol;
-        if (m0 + BM <= args.M && n0 + BN <= args.N) {
+        float *cp = C + mrow * out.ldc + ncol;
+        if (m0 + BM <= out.M && n0 + BN <= out.N) {
 #pragma unroll
             for (int i = 0; i < TM; i++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
-                    float *p = cp + (int64_t)(i * 32 + 8 * (r / 4) + r % 4) * args.ldc;
+                    float *p = cp + (int64_t)(i * 32 + 8 * (r / 4) + r % 4) * out.ldc;
 #pragma unroll
                     for (int j = 0; j < TN; j++) p[j * 32] = acc[i][j][r];
                 }
@@ -575,11 +597,11 @@ struct GemmTile {
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int row = i * 32 + 8 * (r / 4) + r % 4;
-                if (mrow + row >= args.M) continue;
-                float *p = cp + (int64_t)row * args.ldc;
+                if (mrow + row >= out.M) continue;
+                float *p = cp + (int64_t)row * out.ldc;
 #pragma unroll
                 for (int j = 0; j < TN; j++)
-                    if (ncol + j * 32 < args.N) p[j * 32] = acc[i][j][r];
+                    if (ncol + j * 32 < out.N) p[j * 32] = acc[i][j][r];
             }
     }
 };
