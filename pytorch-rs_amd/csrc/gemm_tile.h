@@ -35,7 +35,7 @@
 // The one case behind is an output, or a K slice's part of it, that is a single
 // nonzero product: the three products left out, below 2^-24 of it together,
 // take a diagonal operand from 2.52e-8 to 2.59e-8 (4% of such outputs are the
-// neighbour of the correctly rounded product) and [64, 512] @ [512, 200] in 8
+// neighbour of the correctly rounded product; K = 1 goes to fp32 MFMA) and [64, 512] @ [512, 200] in 8
 // slices with a 0.02 share of nonzeros from 5.52e-8 to 5.58e-8.
 //
 // An output of a tile depends on its row of A and its column of B alone,
@@ -537,29 +537,35 @@ struct GemmTile {
         const int whole = __builtin_amdgcn_readfirstlane((int)(kspan >> 4));
         const int tail = __builtin_amdgcn_readfirstlane((int)(kspan & (kSlot - 1)));
         const gt_flag bad = (gt_flag)(lds + 3 * kBuf);
-        clear();
-        oa.plan(A, args.M - m0, lda, tid);
-        ob.plan(B, args.N - n0, ldb, tid);
-        const uint32_t lost = split_slots(whole, tail, tid, bad);
-        // What follows works its lane values out again, so that the slot loop
-        // does not keep them live.
-        asm volatile("" : "+v"(tid));
-        lane = tid & 63;
-        // A non-finite accumulator leaves a non-finite sum of them.
-        float sum[4] = {0.f, 0.f, 0.f, 0.f};
+        // One k is one product per output, which the split does not always
+        // round correctly (its time is that of the output's store either way).
+        bool fp32 = kspan == 1;
+        if (!fp32) {
+            clear();
+            oa.plan(A, args.M - m0, lda, tid);
+            ob.plan(B, args.N - n0, ldb, tid);
+            const uint32_t lost = split_slots(whole, tail, tid, bad);
+            // What follows works its lane values out again, so that the slot loop
+            // does not keep them live.
+            asm volatile("" : "+v"(tid));
+            lane = tid & 63;
+            // A non-finite accumulator leaves a non-finite sum of them.
+            float sum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < TM; i++)
+            for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int j = 0; j < TN; j++)
+                for (int j = 0; j < TN; j++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    acc[i][j][r] += low[i][j][r];
-                    sum[r & 3] += acc[i][j][r];
-                }
-        const float s = (sum[0] + sum[1]) + (sum[2] + sum[3]);
-        if ((lost & 0xffffu) != 0 || !(__builtin_fabsf(s) < __builtin_inff())) *bad = 1;
-        __syncthreads();
-        if (__builtin_expect(__builtin_amdgcn_readfirstlane(*bad), 0)) {
+                    for (int r = 0; r < 16; r++) {
+                        acc[i][j][r] += low[i][j][r];
+                        sum[r & 3] += acc[i][j][r];
+                    }
+            const float s = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+            if ((lost & 0xffffu) != 0 || !(__builtin_fabsf(s) < __builtin_inff())) *bad = 1;
+            __syncthreads();
+            fp32 = __builtin_amdgcn_readfirstlane(*bad);
+        }
+        if (fp32) {
             clear();
             oa.plan(A, args.M - m0, lda, tid);
             ob.plan(B, args.N - n0, ldb, tid);

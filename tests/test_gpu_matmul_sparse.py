@@ -48,3 +48,13 @@ def test_equal_rows_and_columns_give_equal_bits(m, k, n):
     a, col = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal(k).astype(np.float32)
     got = U.matmul(a.ravel(), (m, k), (k, 1), 0, np.repeat(col, n), (k, n), (n, 1), 0)
     assert np.array_equal(got, np.broadcast_to(got[:, :1], got.shape))
+
+
+@pytest.mark.parametrize("m,n", [(4096, 4096), (1000, 1000), (64, 200)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False)])
+def test_outer_products_are_correctly_rounded(m, n, ta, tb):
+    """K = 1, where an operand's only column may be read as either layout."""
+    rng = np.random.default_rng(m + n)
+    a, b = rng.standard_normal((m, 1)).astype(np.float32), rng.standard_normal((1, n)).astype(np.float32)
+    got = U.matmul(a.ravel(), (m, 1), (1, m) if ta else (1, 1), 0, b.ravel(), (1, n), (1, 1) if tb else (n, 1), 0)
+    assert np.array_equal(got, a * b)
