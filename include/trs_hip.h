@@ -250,8 +250,9 @@ int trs_accumulate_f32(float *dst, const float *src, size_t n);
  * slice's part of it, is a single nonzero product is it not always the
  * correctly rounded one (up to 1.03 times that error, in the 2-norm).  Equal
  * rows of a tile give equal results; A @ A^T need not be symmetric bit for
- * bit.  A tile that holds an infinity, a NaN, a nonzero value below 2^-110
- * with low bits set, or a sum that overflows is computed on fp32 MFMA instead,
+ * bit.  A tile that holds an infinity, a NaN, a sum that overflows, or a
+ * nonzero value below 2^-110 with low bits set that an output may be small
+ * enough to show (2^-32 of it) is computed on fp32 MFMA instead,
  * and so is K = 1.  Outputs with a side of at most 32 use fp32 arithmetic
  * throughout.  Rank 2 ([M,K] @ [K,N]) or rank 3
  * ([b,M,K] @ [b,K,N], the batch the reference spells as rank-2 calls).

@@ -85,11 +85,11 @@ __global__ void __launch_bounds__(T::NT, 1) gemm_split_tile_sk(GemmArgs) {
     const int64_t u0 = b * U / G, u1 = (b + 1) * U / G;
     // Segment: slices [qb, qe) of tile t; the next starts the next tile.
     int64_t t = u0 / Q, qb = u0 - t * Q;
+    T tile((gt_lds)lds);
     for (int64_t u = u0; u < u1; t++, qb = 0) {
         GemmArgsRef args = kernel_args();
         const int64_t qe = imin(Q, qb + (u1 - u));
         float *ws = (qb == 0 && qe == Q) ? nullptr : args.sk_ws + (2 * b + (u == u0 ? 0 : 1)) * kLargeTileFloats;
-        T tile((gt_lds)lds);
         tile.run(args, decode_tile(args, (uint32_t)t), qb * args.sk_depth, qe * args.sk_depth, ws);
         u += qe - qb;
     }

@@ -43,11 +43,16 @@
 // and B, so A @ A.mT is symmetric to rounding only; and a tile that falls back
 // to fp32 MFMA (below) rounds all its outputs as that does.
 //
-// Where the split does not hold -- a value whose lowest bits fall below
-// bf16's smallest subnormal (|x| < 2^-110 with low bits set), an infinity, a
-// NaN, a sum that overflows on the way -- the tile is computed again on fp32
-// MFMA (fp32_slots): the split notes lost bits as it goes, and everything
-// else leaves a non-finite accumulator.
+// Where the split does not hold -- an infinity, a NaN, a sum that overflows on
+// the way, or a value whose lowest bits fall below bf16's smallest subnormal
+// (|x| < 2^-110 with low bits set) and can show in an output -- the part of the
+// tile is computed again on fp32 MFMA (fp32_slots).  The first three leave a
+// non-finite accumulator; the split notes lost bits as it goes, and harmed()
+// bounds what they can do by the rows' largest values, which survey() reads.
+// Lost bits in the first slots of rows that hold nothing larger go to fp32 MFMA
+// at once (useless()).  4096^3, one value of 2^-119 in every 64 rows: 905-935 us
+// (950 on the fp32 MFMA build; 1,630 where every such tile was computed
+// again), all values that small: 1,110-1,140 (950; 1,590).
 //
 // What bounds it: the card's power.  At 4096^3 random values run 640-670 us
 // (1,230-1,290 TFLOP/s of bf16), zeros in far less at a higher clock.  The fp32
@@ -68,7 +73,7 @@ typedef const float __attribute__((address_space(1))) *gt_global;
 typedef const char __attribute__((address_space(1))) *gt_global_bytes;
 typedef char __attribute__((address_space(3))) *gt_lds;
 typedef float __attribute__((address_space(3))) *gt_lds_floats;
-typedef volatile int __attribute__((address_space(3))) *gt_flag;
+typedef uint32_t __attribute__((address_space(3))) *gt_lds_words;
 typedef __bf16 gt_bf2 __attribute__((ext_vector_type(2)));
 typedef __bf16 gt_bf8 __attribute__((ext_vector_type(8)));
 
@@ -103,6 +108,10 @@ __device__ __forceinline__ GemmArgsRef kernel_args() {
     asm volatile("" : "+s"(p));
     return *p;
 }
+
+// Floats below this (2^-110) have bits below bf16's smallest subnormal, 2^-133;
+// what the split loses of one is at most half of that.
+constexpr uint32_t kTiny = (127u - 110u) << 23;
 
 constexpr int kGroupM = 8;
 constexpr int kXcds = 8;
@@ -278,6 +287,18 @@ struct SlotOperand {
             *(PackLds)(d + 2 * kPlane) = l;
         }
     }
+    // For each chunk, as floats: the largest |value| so far, and 1 if a value was
+    // one whose split may lose bits.
+    __device__ __forceinline__ void note(const Regs &v, uint32_t (&most)[NC], uint32_t (&tiny)[NC]) const {
+#pragma unroll
+        for (int q = 0; q < NC; q++)
+#pragma unroll
+            for (int e = 0; e < CH; e++) {
+                const uint32_t u = __float_as_uint(v[q][e]) & 0x7fffffffu;
+                most[q] = most[q] > u ? most[q] : u;
+                if (u - 1 < kTiny - 1) tiny[q] = 0x3f800000u;
+            }
+    }
     // As floats, [k][row]: the pitch puts k and k + 1 half the banks apart.
     __device__ __forceinline__ void store_fp32(const Regs &v, gt_lds_floats lds) const {
 #pragma unroll
@@ -296,8 +317,10 @@ struct GemmTile {
     using OA = SlotOperand<BM, NT, AKC>;
     using OB = SlotOperand<BN, NT, BKC>;
     static constexpr int kABytes = 3 * OA::kPlane, kBuf = kABytes + 3 * OB::kPlane;
-    // Three slots in LDS, and the flag of a tile the split does not hold for.
-    static constexpr int kLds = 3 * kBuf + 16;
+    // Three slots in LDS, a word a wave for each of three notices, and survey()'s values.
+    enum Notice { kFirstLost, kResult, kFails };
+    static constexpr int NW = WGM * WGN, kNotices = 3 * kBuf;
+    static constexpr int kSurvey = kNotices + 3 * NW * 4, kLds = kSurvey + 2 * (BM + BN) * 4;
     static constexpr int kFp32A = kSlot * OA::kPitch, kFp32Buf = kFp32A + kSlot * OB::kPitch;
     static_assert(2 * kFp32Buf * 4 <= 3 * kBuf, "the fp32 slots fit the split ones' LDS");
     static_assert(AHEAD == 1 || AHEAD == 2, "the slot loop is unrolled over two register sets");
@@ -313,13 +336,30 @@ struct GemmTile {
 
     __device__ __forceinline__ explicit GemmTile(gt_lds l) : lds(l) {}
 
+    // What the waves of a block tell one another: each posts a word (the same in
+    // all its lanes) ahead of a barrier, and reads the or of them behind it.  All
+    // post every time, so nothing has to be cleared.
+    __device__ __forceinline__ void post(Notice n, uint32_t word, unsigned tid) const {
+        ((gt_lds_words)(lds + kNotices))[n * NW + (tid >> 6)] = word;
+    }
+    __device__ __forceinline__ uint32_t posted(Notice n) const {
+        uint32_t any = 0;
+#pragma unroll
+        for (int w = 0; w < NW; w++) any |= ((gt_lds_words)(lds + kNotices))[n * NW + w];
+        return __builtin_amdgcn_readfirstlane(any);
+    }
+    // Whether a condition holds in a lane of this wave.
+    __device__ __forceinline__ static bool in_wave(bool lane) { return __builtin_amdgcn_ballot_w64(lane) != 0; }
+
     __device__ __forceinline__ void clear() {
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int j = 0; j < TN; j++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) acc[i][j][r] = low[i][j][r] = 0.f;
+            for (int j = 0; j < TN; j++) {
+                acc[i][j] = low[i][j] = (gt_f16)(0.f);
+                // Here, and not where they are first used.
+                asm volatile("" : "+v"(acc[i][j]), "+v"(low[i][j]));
+            }
     }
     struct Slot {  // a slot's floats on their way to LDS
         typename OA::Regs a;
@@ -343,8 +383,8 @@ struct GemmTile {
     // the next row, and the slot's splitting and loads, sit among the MFMAs
     // of the row before.  Loads past the last slot repeat it (a branch around
     // a load makes the compiler wait for every load at the join).
-    __device__ __forceinline__ uint32_t split_slots(int whole, int tail, unsigned tid, gt_flag bad) {
-        uint32_t lost = 0;
+    __device__ __forceinline__ bool split_slots(int whole, int tail, unsigned tid, uint32_t &lost) {
+        lost = 0;
         Slot in[AHEAD];
         const int T = whole + (tail ? 1 : 0);
         int left = whole;  // whole slots not yet loaded
@@ -356,11 +396,6 @@ struct GemmTile {
         const auto put = [&](const Slot &r, int buf) {
             oa.store_split(r.a, lds + buf, lost);
             ob.store_split(r.b, lds + buf + kABytes, lost);
-        };
-        // After the prologue: every wave is done with the tile before, the flag included.
-        const auto ready = [&]() {
-            __syncthreads();
-            if (tid == 0) *bad = 0;
         };
         typedef const gt_bf8 __attribute__((address_space(3))) *Frag;
         const gt_lds fa = lds + wm0 * 32 + lane * 16, fb = lds + kABytes + wn0 * 32 + lane * 16;
@@ -415,10 +450,27 @@ struct GemmTile {
             const int c = cur;
             cur = nxt, nxt = wr, wr = c;
         };
-        const auto first = [&]() {
+        // The first slots are in LDS: the first fragments, and whether to give up.
+        const auto first = [&](int slots, const Slot &s0, const Slot &s1) {
+            post(kFirstLost, in_wave((lost & 0xffffu) != 0), tid);
+            __syncthreads();
             read_a(0, 0, A[0]);
 #pragma unroll
             for (int j = 0; j < TN; j++) read_b(0, j);
+            const uint32_t any = posted(kFirstLost);
+            // All of these reads are out before the branch.
+#pragma unroll
+            for (int p = 0; p < 3; p++) {
+                asm volatile("" : "+v"(A[0][p]));
+#pragma unroll
+                for (int j = 0; j < TN; j++) asm volatile("" : "+v"(B[j][p]));
+            }
+            if (__builtin_expect(!any, 1)) return false;
+            Extremes x = {};
+            note(s0, x);
+            if (slots > 1) note(s1, x);
+            merge(x, tid);
+            return useless(tid);
         };
         // The first slots' loads all go out together.
         Slot s0, s1;
@@ -431,11 +483,11 @@ struct GemmTile {
             ta.load_tail(s0.a, lda, tail);
             tb.load_tail(s0.b, ldb, tail);
             if (!whole) {
+                clear();
                 put(s0, 0);
-                ready();
-                first();
+                if (__builtin_expect(first(1, s0, s0), 0)) return true;
                 slot.template operator()<false, 0>();
-                return lost;
+                return false;
             }
         } else {
             load(s0);
@@ -448,10 +500,10 @@ struct GemmTile {
             load(in[d]);
             move_on();
         }
+        clear();  // under the loads
         put(s0, 0);
         put(s1, kBuf);
-        ready();
-        first();
+        if (__builtin_expect(first(2, s0, s1), 0)) return true;
         // Slot t takes registers t % AHEAD.
         int t = 0;
 #pragma unroll 1
@@ -460,7 +512,89 @@ struct GemmTile {
             slot.template operator()<true, 1 % AHEAD>();
         }
         if (t < T) slot.template operator()<true, 0>();
-        return lost;
+        return false;
+    }
+
+    // What lost bits can do: every row of A's and column of B's largest |value|
+    // and whether (1 or 0) it holds a tiny one, per lane and then into LDS.
+    struct Extremes {
+        uint32_t most_a[OA::NC], tiny_a[OA::NC], most_b[OB::NC], tiny_b[OB::NC];
+    };
+    __device__ __forceinline__ void note(const Slot &s, Extremes &x) const {
+        oa.note(s.a, x.most_a, x.tiny_a);
+        ob.note(s.b, x.most_b, x.tiny_b);
+    }
+    __device__ __forceinline__ void merge(const Extremes &x, unsigned tid) const {
+        const gt_lds_words most = (gt_lds_words)(lds + kSurvey), tiny = most + BM + BN;
+        for (int i = tid; i < 2 * (BM + BN); i += NT) most[i] = 0;
+        __syncthreads();
+        const auto raise = [](gt_lds_words p, uint32_t v) {
+            __hip_atomic_fetch_max(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        };
+#pragma unroll
+        for (int q = 0; q < OA::NC; q++) raise(most + oa.row[q], x.most_a[q]), raise(tiny + oa.row[q], x.tiny_a[q]);
+#pragma unroll
+        for (int q = 0; q < OB::NC; q++)
+            raise(most + BM + ob.row[q], x.most_b[q]), raise(tiny + BM + ob.row[q], x.tiny_b[q]);
+        __syncthreads();
+    }
+    // Of all slots, four on their way at a time.
+    __device__ __forceinline__ void survey(int whole, int tail, unsigned tid) {
+        Extremes x = {};
+        Slot in[4];
+        const auto move_on = [&]() {
+            oa.advance(astep);
+            ob.advance(bstep);
+        };
+        int t = 0;
+#pragma unroll 1
+        for (; t + 4 <= whole; t += 4) {
+#pragma unroll
+            for (int d = 0; d < 4; d++) load(in[d]), move_on();
+#pragma unroll
+            for (int d = 0; d < 4; d++) note(in[d], x);
+        }
+#pragma unroll 1
+        for (; t < whole; t++) load(in[0]), move_on(), note(in[0], x);
+        if (tail) {
+            oa.load_tail(in[0].a, lda, tail);
+            ob.load_tail(in[0].b, ldb, tail);
+            note(in[0], x);
+        }
+        merge(x, tid);
+    }
+    // After survey(): whether lost bits may show in one of this lane's outputs.
+    // The split is off by at most 2^-134 in a tiny value, so an output by that
+    // times the other operand's values.  Up to 2^-32 of the output it is 2^-8
+    // of a rounding.
+    static constexpr float kLeast = 0x1p-102f;
+    __device__ __forceinline__ bool harmed(int whole, int tail) const {
+        const gt_lds_floats most = (gt_lds_floats)(lds + kSurvey), tiny = most + BM + BN;
+        const float scale = (float)(whole * kSlot + tail) * kLeast;
+        float worst = 0.f;
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            const int col = BM + wn0 + j * 32 + (lane & 31);
+            const float mb = scale * most[col], tb = scale * tiny[col];
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int row = wm0 + i * 32 + 8 * (r / 4) + 4 * (lane >> 5) + r % 4;
+                    worst = __builtin_fminf(worst, __builtin_fabsf(acc[i][j][r]) - (tiny[row] * mb + most[row] * tb));
+                }
+        }
+        return worst < 0.f;
+    }
+    // After merge() of the first slots: whether none of a row's (column's) outputs
+    // is likely to pass that, its values so far being too small.
+    __device__ __forceinline__ bool useless(unsigned tid) const {
+        const gt_lds_floats most = (gt_lds_floats)(lds + kSurvey), tiny = most + BM + BN;
+        bool none = false;
+        for (int i = tid; i < BM + BN; i += NT) none |= tiny[i] != 0.f && most[i] < kLeast;
+        post(kFails, in_wave(none), tid);
+        __syncthreads();
+        return posted(kFails);
     }
 
     // The same slots on fp32 MFMA (v_mfma_f32_32x32x2_f32), double-buffered.
@@ -528,47 +662,61 @@ struct GemmTile {
         wm0 = (wave / WGN) * WM;
         wn0 = (wave % WGN) * WN;
         const int64_t Kb = args.ktotal ? imin(args.K, args.ktotal - batch * args.K) : args.K;
-        const float *A = args.a + batch * args.bsa + (AKC ? m0 * lda + k0 : m0 + k0 * lda);
-        const float *B = args.b + batch * args.bsb + (BKC ? n0 * ldb + k0 : n0 + k0 * ldb);
         astep = AKC ? kSlot : kSlot * lda;
         bstep = BKC ? kSlot : kSlot * ldb;
         const int64_t kspan = imin(k1, Kb) - k0;
         // 64-bit compares run on the vector units; back to scalar registers.
         const int whole = __builtin_amdgcn_readfirstlane((int)(kspan >> 4));
         const int tail = __builtin_amdgcn_readfirstlane((int)(kspan & (kSlot - 1)));
-        const gt_flag bad = (gt_flag)(lds + 3 * kBuf);
+        const auto to_first = [&](GemmArgsRef g) {
+            const float *A = g.a + batch * g.bsa + (AKC ? m0 * lda + k0 : m0 + k0 * lda);
+            const float *B = g.b + batch * g.bsb + (BKC ? n0 * ldb + k0 : n0 + k0 * ldb);
+            oa.plan(A, g.M - m0, lda, tid);
+            ob.plan(B, g.N - n0, ldb, tid);
+        };
+        to_first(args);
         // One k is one product per output, which the split does not always
         // round correctly (its time is that of the output's store either way).
         bool fp32 = kspan == 1;
-        if (!fp32) {
-            clear();
-            oa.plan(A, args.M - m0, lda, tid);
-            ob.plan(B, args.N - n0, ldb, tid);
-            const uint32_t lost = split_slots(whole, tail, tid, bad);
+        if (__builtin_expect(!fp32, 1)) {
+            uint32_t lost;
+            fp32 = split_slots(whole, tail, tid, lost);
             // What follows works its lane values out again, so that the slot loop
             // does not keep them live.
             asm volatile("" : "+v"(tid));
             lane = tid & 63;
-            // A non-finite accumulator leaves a non-finite sum of them.
-            float sum[4] = {0.f, 0.f, 0.f, 0.f};
+            if (__builtin_expect(!fp32, 1)) {
+                // A non-finite accumulator leaves a non-finite sum of them.
+                float sum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int i = 0; i < TM; i++)
+                for (int i = 0; i < TM; i++)
 #pragma unroll
-                for (int j = 0; j < TN; j++)
+                    for (int j = 0; j < TN; j++)
 #pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        acc[i][j][r] += low[i][j][r];
-                        sum[r & 3] += acc[i][j][r];
-                    }
-            const float s = (sum[0] + sum[1]) + (sum[2] + sum[3]);
-            if ((lost & 0xffffu) != 0 || !(__builtin_fabsf(s) < __builtin_inff())) *bad = 1;
-            __syncthreads();
-            fp32 = __builtin_amdgcn_readfirstlane(*bad);
+                        for (int r = 0; r < 16; r++) {
+                            acc[i][j][r] += low[i][j][r];
+                            sum[r & 3] += acc[i][j][r];
+                        }
+                const float s = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+                const bool bad = !(__builtin_fabsf(s) < __builtin_inff());
+                post(kResult, in_wave((lost & 0xffffu) != 0) | in_wave(bad) << 1, tid);
+                __syncthreads();
+                const uint32_t result = posted(kResult);
+                fp32 = result & 2;
+                if (__builtin_expect(result == 1, 0)) {
+                    to_first(kernel_args());
+                    int slots = whole, rest = tail;  // nothing of this ahead of the slot loop
+                    asm volatile("" : "+s"(slots), "+s"(rest));
+                    survey(slots, rest, tid);
+                    post(kFails, in_wave(harmed(slots, rest)), tid);
+                    __syncthreads();
+                    fp32 = posted(kFails);
+                }
+            }
+            if (__builtin_expect(fp32, 0)) to_first(kernel_args());
         }
-        if (fp32) {
+        if (__builtin_expect(fp32, 0)) {
             clear();
-            oa.plan(A, args.M - m0, lda, tid);
-            ob.plan(B, args.N - n0, ldb, tid);
             fp32_slots(whole, tail);
         }
         GemmArgsRef out = PARTS == 1 ? args : kernel_args();
