@@ -153,3 +153,33 @@ def test_stride_0_and_long_row_strides():
     far.reshape(m, 5003)[:, 3:3 + k] = a
     got = U.matmul(far, (m, k), (5003, 1), 3, b.ravel(), (k, n), (n, 1), 0)
     assert np.array_equal(got.reshape(m, n), a @ b)
+
+
+@pytest.mark.parametrize("m,k,n", [(4096, 100, 4096), (1000, 1000, 1000), (512, 4096, 4096), (70, 120, 200)])
+@pytest.mark.parametrize("right", [False, True])
+def test_sums_that_overflow(m, k, n, right):
+    """Values whose pieces are finite, and whose sums reach float's largest.  v is
+    the float below 2^127: 2 v is the largest float, and the leading pieces of
+    two v (2^127 each) add up to infinity, which fp32 arithmetic does not.  On
+    one tile, in K slices and in stream-K's pieces; the other operand is ones."""
+    v = np.nextafter(np.float32(2.0 ** 127), np.float32(0))
+    top, inf = np.finfo(np.float32).max, np.float32(np.inf)
+    at = [3, 5, k // 2, k - 9, k - 1]  # a group of 8 k, others, the last one
+    rows, want = [], []
+    for i in range(5):
+        for j in range(i):
+            rows += [{at[i]: v, at[j]: v}, {at[i]: -v, at[j]: -v}]
+            want += [top, -top]
+    rows += [{p: v for p in at[:3]}, {p: v for p in at[2:]}, {p: -v for p in at[::2]}]
+    want += [inf, inf, -inf]
+    x = np.zeros((n if right else m, k), np.float32)
+    expected = np.zeros(x.shape[0], np.float32)
+    for i, (row, w) in enumerate(zip(rows, want)):
+        x[7 + 2 * i, list(row)] = list(row.values())
+        expected[7 + 2 * i] = w
+    back = 7 + 2 * len(rows)
+    x[back, at] = [v, v, -v, -v, v]  # 2 v on the way, v in the end, in whatever order
+    expected[back] = v
+    other = np.ones((k, m if right else n), np.float32)
+    got = _product(other.T, x.T, False, False).T if right else _product(x, other, False, False)
+    assert np.array_equal(got, np.broadcast_to(expected[:, None], got.shape))
