@@ -504,27 +504,30 @@ bool reduce_cols_plan(const ReduceGeom &rg, bool has_other, RedColsGeom *cg) {
 }
 
 // Whether the staged kernel is the faster one for cg's chains: up to a number
-// of chains that grows with their length.  A staged block costs about 4.5 us
-// whatever its rows, and its blocks run in rounds; the unrolled kernel costs a
-// memory latency per 8 rows, with any number of chains, until it is bound by
-// memory.  Measured, staged / unrolled, in us:
-//   rows   chains per CU
-//     16   32: 5.4 / 6.7      64: 7.4 / 6.6
-//     64   64: 7.6 / 7.8     128: 11.7 / 8.1
-//    128  128: 13.8 / 15.3   256: 23.1 / 15.6
-//    255  128: 19.9 / 28.0   256: 34.1 / 28.3
-//    400  256: 38.7 / 50.3   512: 72.0 / 57.5
-//   1000  256: 77.3 / 123    512: 147 / 138
+// of blocks that grows with the chains' length.  A staged block costs its
+// stages whether all of its 32 chains are there or 4 (a KI that is no multiple
+// of 32 leaves some idle, in each of KO blocks), and its blocks run in rounds;
+// the unrolled kernel costs a memory latency per 8 rows, with any number of
+// chains, until it is bound by memory.  Measured, staged / unrolled, in us, at
+// KI = 4, 17 and 100 (unaligned rows):
+//   rows  blocks per CU
+//     16    1: 3.9/4.8  4.1/4.7  4.0/4.8       2: 5.5/4.8  5.5/4.6  5.5/4.8
+//     64    2: 5.6/7.7  5.6/7.9  5.6/8.0       4: 9.7/7.7  9.8/7.9  9.8/8.0
+//    128    4: 10.7/12.2 10.9/12.6 11.1/13.8   8: 19.9/12.3 20.4/15.5 21.8/15.3
+//    256    4: 11.6/21.9 11.9/22.6 15.5/27.2   8: 21.7/22.0 22.4/28.5 28.5/28.4
+//    512   14: 37.5/41.2 40.6/54.4 56.5/56.2  20: 52.5/49.0 56.9/56.1 77.8/57.6
+//   1000   14: 65.0/94.7 69.4/104 111/133     20: 91.6/95.4 99.2/141 154/141
+// ([28000, 1000, 4] summed over its rows, 109 blocks per CU: 492 staged, 140
+// unrolled; [8192, 1000] -> [1000] 32.6 staged, 796 unrolled.)
 // Chains that start and stay 16-byte aligned, in whole blocks, read faster
 // ([1000, 65536] 64 us): staged from 256 rows on, whatever their number.
-// (A gradient [8192, 1000] -> [1000] took 796 us unrolled, 32.6 staged.)
 constexpr int64_t kStMinRows = 16;
 
 bool staged_pays(const RedColsGeom &cg, bool whole_aligned, int cu_count) {
     if (cg.R < kStMinRows) return false;
     if (whole_aligned && cg.R >= kStRows) return true;
-    const int64_t per_cu = cg.R < 64 ? 32 : cg.R < 128 ? 64 : cg.R < 256 ? 128 : cg.R < 512 ? 256 : 448;
-    return cg.KO * cg.KI <= per_cu * cu_count;
+    const int64_t per_cu = cg.R < 64 ? 1 : cg.R < 128 ? 2 : cg.R < 256 ? 4 : cg.R < 512 ? 7 : 14;
+    return cg.KO * ((cg.KI + kStChains - 1) / kStChains) <= per_cu * cu_count;
 }
 
 int reduce_to_operand(const float *up, const trs_layout *lout, const float *other,

@@ -4,6 +4,7 @@ is added in the reference's order from +0.0, so results equal a sequential
 float32 sum bit for bit.
 """
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -65,3 +66,40 @@ def test_broadcast_mul_gradients_of_any_width(nb, rows, cols, kind):
     for r in range(rows):
         want += prod[:, r]
     _same(do.to_numpy(count=nb * cols).reshape(nb, cols), want)
+
+
+# Many outer kept indices of a few columns each, on both sides of the number of
+# blocks (one per outer index and 32 columns, whole or not) up to which the staged
+# kernel is taken on a 256-CU device: 1, 2, 4, 7 and 14 per CU.
+@pytest.mark.parametrize("ko,rows,ki", [(256, 20, 4), (257, 20, 4), (256, 65, 33), (257, 65, 33), (1024, 130, 8),
+                                        (1025, 130, 8), (1792, 260, 5), (1793, 260, 5), (3584, 513, 4), (3585, 513, 4),
+                                        (1792, 513, 40), (1793, 513, 40)])
+def test_broadcast_gradients_of_many_narrow_groups(ko, rows, ki):
+    rng = np.random.default_rng(ko + rows + ki)
+    up = _normal(rng, ko, rows, ki)
+    du, do = U.dev(up), U.out_buffer(ko * ki)
+    check(abi.lib.trs_reduce_to_shape_f32(du.ptr, ctypes.byref(layout_of((ko, rows, ki))),
+                                          ctypes.byref(layout_of((ko, 1, ki))), do.ptr))
+    want = np.zeros((ko, ki), np.float32)
+    for r in range(rows):
+        want += up[:, r]
+    _same(do.to_numpy(count=ko * ki).reshape(ko, ki), want)
+
+
+def test_narrow_groups_take_no_longer_than_twice_one_wide_one():
+    """The same chains as 28,000 groups of 4 and as one of 112,000: 140 and about
+    90 us (492 where 28,000 staged blocks each add 4 chains)."""
+    up, out = U.out_buffer(112000 * 1000, 1.0), U.out_buffer(112000)
+
+    def best(shape, kept):
+        lu, ls, times = layout_of(shape), layout_of(kept), []
+        for _ in range(8):
+            check(abi.lib.trs_synchronize())
+            t = time.perf_counter()
+            for _ in range(10):
+                check(abi.lib.trs_reduce_to_shape_f32(up.ptr, ctypes.byref(lu), ctypes.byref(ls), out.ptr))
+            check(abi.lib.trs_synchronize())
+            times.append(time.perf_counter() - t)
+        return min(times)
+
+    assert best((28000, 1000, 4), (28000, 1, 4)) < 2.5 * best((1000, 112000), (112000,))
