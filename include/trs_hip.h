@@ -319,7 +319,7 @@ typedef struct trs_pw_plan_info {
     int32_t variant;    /* 0 nothing to do, 1 flat, 2 rows, 3 transposing, 4 generic */
     int32_t rank;       /* rank after dropping size-1 dims and merging contiguous ones */
     int32_t vec;        /* 16-byte vector accesses, all of them 16-byte aligned
-                         * (0: at any float, or scalar) */
+                         * (0: at any float, or scalar: trs_pointwise_plan_access) */
     int32_t fixed_rank; /* rank the kernel is compiled for (32-bit offsets), 0 = decoded at run time */
     int32_t skew;       /* transposing: a tuple's tiles taken in diagonal order */
     int32_t walk;       /* transposing: outer tuples per block */
@@ -336,6 +336,13 @@ typedef struct trs_pw_plan_info {
 int trs_pointwise_plan(int n_inputs, const void *const *inputs, const trs_layout *const *layouts,
                        const int *elem_bytes, const float *out, const trs_layout *lo, int cu_count, int roles,
                        trs_pw_plan_info *info);
+/* How the kernel of that plan reaches memory: *vector, with 16-byte vectors
+ * (whatever their alignment; 0: element by element), and *through_lds, the
+ * transposing kernel that turns its tiles through LDS.  Arguments and errors as
+ * above; either out pointer may be null. */
+int trs_pointwise_plan_access(int n_inputs, const void *const *inputs, const trs_layout *const *layouts,
+                              const int *elem_bytes, const float *out, const trs_layout *lo, int cu_count, int roles,
+                              int *vector, int *through_lds);
 
 /* ---- pointwise fusion compiler (new; no counterpart in the reference) */
 

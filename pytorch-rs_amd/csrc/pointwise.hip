@@ -776,6 +776,23 @@ int sum_launch(DeviceState *dev, const float *x, const trs_layout *lx, float *ou
 
 using namespace trs;
 
+namespace {
+
+// The plan that the diagnostics report, and their checks.
+int report_plan(int n_inputs, const void *const *inputs, const trs_layout *const *layouts, const int *elem_bytes,
+                const float *out, const trs_layout *lo, int cu_count, int roles, PwPlan *pl) {
+    if (n_inputs < 1 || n_inputs > kMaxIn)
+        return set_error(TRS_E_INVALID_ARGUMENT, "pointwise plans take 1 to %d inputs, got %d", kMaxIn, n_inputs);
+    if (!inputs || !layouts) return set_error(TRS_E_INVALID_ARGUMENT, "null input arrays");
+    if (cu_count < 1) return set_error(TRS_E_INVALID_ARGUMENT, "cu_count must be positive, got %d", cu_count);
+    int eb[kMaxIn];
+    for (int i = 0; i < n_inputs; i++) eb[i] = elem_bytes ? elem_bytes[i] : 4;
+    return plan_pointwise(lo, const_cast<float *>(out), n_inputs, inputs, layouts, eb, cu_count, pl, 1, nullptr,
+                          roles != 0);
+}
+
+}  // namespace
+
 extern "C" {
 
 int trs_accumulate_f32(float *dst, const float *src, size_t n) {
@@ -839,15 +856,8 @@ int trs_pointwise_plan(int n_inputs, const void *const *inputs, const trs_layout
                        const int *elem_bytes, const float *out, const trs_layout *lo, int cu_count, int roles,
                        trs_pw_plan_info *info) {
     if (!info) return set_error(TRS_E_INVALID_ARGUMENT, "null plan info");
-    if (n_inputs < 1 || n_inputs > kMaxIn)
-        return set_error(TRS_E_INVALID_ARGUMENT, "pointwise plans take 1 to %d inputs, got %d", kMaxIn, n_inputs);
-    if (!inputs || !layouts) return set_error(TRS_E_INVALID_ARGUMENT, "null input arrays");
-    if (cu_count < 1) return set_error(TRS_E_INVALID_ARGUMENT, "cu_count must be positive, got %d", cu_count);
-    int eb[kMaxIn];
-    for (int i = 0; i < n_inputs; i++) eb[i] = elem_bytes ? elem_bytes[i] : 4;
     PwPlan pl;
-    const int rc = plan_pointwise(lo, const_cast<float *>(out), n_inputs, inputs, layouts, eb, cu_count, &pl, 1,
-                                  nullptr, roles != 0);
+    const int rc = report_plan(n_inputs, inputs, layouts, elem_bytes, out, lo, cu_count, roles, &pl);
     if (rc) return rc;
     *info = trs_pw_plan_info{};
     info->variant = (int32_t)pl.variant;
@@ -866,6 +876,17 @@ int trs_pointwise_plan(int n_inputs, const void *const *inputs, const trs_layout
     int64_t launches = pl.variant == PwVariant::Empty ? 0 : 1;
     for (int d = 0; d < pl.nsplit; d++) launches = std::min<int64_t>(launches * pl.ssize[d], INT32_MAX);
     info->launches = (int32_t)launches;
+    return TRS_OK;
+}
+
+int trs_pointwise_plan_access(int n_inputs, const void *const *inputs, const trs_layout *const *layouts,
+                              const int *elem_bytes, const float *out, const trs_layout *lo, int cu_count, int roles,
+                              int *vector, int *through_lds) {
+    PwPlan pl;
+    const int rc = report_plan(n_inputs, inputs, layouts, elem_bytes, out, lo, cu_count, roles, &pl);
+    if (rc) return rc;
+    if (vector) *vector = pl.vec;
+    if (through_lds) *through_lds = pl.lds;
     return TRS_OK;
 }
 

@@ -135,6 +135,8 @@ _SIGNATURES = {
                              POINTER(c_int), POINTER(ctypes.c_int64), POINTER(ctypes.c_int64)], c_int),
     "trs_pointwise_plan": ([c_int, POINTER(c_void_p), POINTER(_LP), POINTER(c_int), c_void_p, _LP, c_int, c_int,
                             POINTER(PwPlanInfo)], c_int),
+    "trs_pointwise_plan_access": ([c_int, POINTER(c_void_p), POINTER(_LP), POINTER(c_int), c_void_p, _LP, c_int, c_int,
+                                   POINTER(c_int), POINTER(c_int)], c_int),
     "trs_fusion_compile": ([c_char_p, c_size_t, POINTER(c_uint64)], c_int),
     "trs_fusion_launch": ([c_uint64, c_int, POINTER(c_void_p), _LP, c_void_p, _LP], c_int),
     "trs_fusion_launch_multi": ([c_uint64, c_int, POINTER(c_void_p), _LP, c_int, POINTER(c_void_p), _LP], c_int),
@@ -174,21 +176,34 @@ def check(rc: int) -> None:
         raise TrsError(rc, msg.decode() if msg else "")
 
 
-def pointwise_plan(layouts, out_layout, bases=None, out=0x10000000000, elem_bytes=None, cu_count=256,
-                   roles=False) -> PwPlanInfo:
-    """trs_pointwise_plan for input `layouts` and `out_layout` (no device
-    needed).  `bases` and `out` are addresses, used only for alignment and
-    the overlap checks: by default far apart and 256-byte aligned."""
+def _plan_arguments(layouts, out_layout, bases, out, elem_bytes, cu_count, roles):
     n = len(layouts)
     if bases is None:
         bases = [0x20000000000 + i * 0x10000000000 for i in range(n)]
     ptrs = (c_void_p * n)(*bases)
     lays = (_LP * n)(*[ctypes.pointer(l) for l in layouts])
     eb = (c_int * n)(*(elem_bytes or [4] * n))
+    return n, ptrs, lays, eb, c_void_p(out), ctypes.byref(out_layout), cu_count, 1 if roles else 0
+
+
+def pointwise_plan(layouts, out_layout, bases=None, out=0x10000000000, elem_bytes=None, cu_count=256,
+                   roles=False) -> PwPlanInfo:
+    """trs_pointwise_plan for input `layouts` and `out_layout` (no device
+    needed).  `bases` and `out` are addresses, used only for alignment and
+    the overlap checks: by default far apart and 256-byte aligned."""
     info = PwPlanInfo()
-    check(lib.trs_pointwise_plan(n, ptrs, lays, eb, c_void_p(out), ctypes.byref(out_layout), cu_count,
-                                 1 if roles else 0, ctypes.byref(info)))
+    check(lib.trs_pointwise_plan(*_plan_arguments(layouts, out_layout, bases, out, elem_bytes, cu_count, roles),
+                                 ctypes.byref(info)))
     return info
+
+
+def pointwise_plan_access(layouts, out_layout, bases=None, out=0x10000000000, elem_bytes=None, cu_count=256,
+                          roles=False) -> tuple[bool, bool]:
+    """trs_pointwise_plan_access: (vector, through_lds) of that plan's kernel."""
+    vector, lds = c_int(), c_int()
+    check(lib.trs_pointwise_plan_access(*_plan_arguments(layouts, out_layout, bases, out, elem_bytes, cu_count, roles),
+                                        ctypes.byref(vector), ctypes.byref(lds)))
+    return bool(vector.value), bool(lds.value)
 
 
 def device_count() -> int:

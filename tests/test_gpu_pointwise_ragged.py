@@ -95,6 +95,32 @@ def test_transposed_operand_at_every_edge(nb, t, x):
     _same(torch_rs.fuse(lambda p, q: p * q)(torch_rs.tensor(col, device="cuda"), dc.mT).numpy(), col * ct)
 
 
+# Those that run on the tiles through LDS (64 t by 256 x, at least 0.55 full):
+# t and x around the tiles' edges, a last tile of one row or column, every
+# residue mod 4, and the least full.
+THROUGH_LDS = [(2, 130, 1001), (2, 36, 253), (1, 64, 144), (1, 64, 145), (3, 63, 146), (1, 63, 147), (1, 62, 255),
+               (2, 64, 254), (1, 129, 1023), (1, 130, 1021), (2, 131, 1022), (1, 64, 769), (1, 64, 770), (1, 64, 771),
+               (1, 127, 511), (2, 125, 700), (3, 128, 510)]
+
+
+@pytest.mark.parametrize("nb,t,x", THROUGH_LDS)
+def test_lds_tiles_at_every_edge(nb, t, x):
+    import torch_rs
+    lays = [layout_of((nb, 1, x)), layout_of((1, t, x)), layout_of((nb, t, x), (t * x, 1, t))]
+    assert abi.pointwise_plan_access(lays, layout_of((nb, t, x)), roles=True) == (True, True)
+    rng = np.random.default_rng(nb + 3 * t + 7 * x)
+    a, b, c = _normal(rng, nb, 1, x), _normal(rng, 1, t, x), _normal(rng, nb, x, t)
+    da, db, dc = (torch_rs.tensor(v, device="cuda") for v in (a, b, c))
+    ct, full = c.transpose(0, 2, 1), a + b
+    _same(torch_rs.fuse(lambda p, q, r: (p + q) * r)(da, db, dc.mT).numpy(), full * ct)
+    _same((torch_rs.tensor(full, device="cuda") + dc.mT).numpy(), full + ct)
+    col, scalar = _normal(rng, nb, t, 1), _normal(rng, 1)
+    dcol, ds = torch_rs.tensor(col, device="cuda"), torch_rs.tensor(scalar, device="cuda")
+    # five inputs: the others are read after the barrier
+    five = torch_rs.fuse(lambda p, q, r, u, v: ((p + q) * r - u) * v)
+    _same(five(da, db, dc.mT, dcol, ds).numpy(), (full * ct - col) * scalar)
+
+
 def test_transposed_views_at_any_float_and_higher_rank():
     import torch_rs
     rng = np.random.default_rng(4)
