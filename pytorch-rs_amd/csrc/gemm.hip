@@ -18,9 +18,10 @@
 //   64x128   4 waves of 32x64, two blocks per CU
 // The 4-wave 128x128 tile reads a third less from LDS per product, which
 // counts where the whole chip runs it and power sets the clock (batched
-// 32x512^3 52.3 us against 54.0, 1000x2047x1500 48.4 against 50.3); the 8-wave
-// one issues its slot in half the instructions per wave, which counts where
-// one block has a CU to itself (700^3 16.6 us against 18.8).
+// 32x512^3 57.6 us against 61.6, 1000x2047x1500 52.6 against 58.7, on one
+// card); the 8-wave one issues its slot in half the instructions per wave, which
+// counts where one block has a CU to itself (700^3 17.6 us against 19.6,
+// 2048x100x2048 12.6 against 13.1).
 // Blocks are remapped so that consecutive tiles share an XCD (each XCD has
 // its own L2), and tiles are walked in groups of kGroupM tile rows.
 #include <hip/hip_runtime.h>
@@ -46,12 +47,11 @@ using MediumTile = GemmTile<64, 128, 2, 2, 2, AKC, BKC>;
 constexpr int64_t kLarge = 256;
 constexpr int64_t kLargeTileFloats = kLarge * kLarge;
 
-// The k a product is dealt out in (a split K's slices are whole multiples,
-// stream-K's units one each): two slots where A is contiguous along k and a
-// long K is whole pairs of slots, else one.
+// The k that stream-K's units hold: two slots where A is contiguous along k and
+// a long K is whole pairs of slots, else one.  The tile takes either alike
+// (512x4096x4096, 3072^3 and 5120^3 within 0.3%); the plan reports it.
 inline int slice_depth(const GemmArgs &g, bool a_plain) {
-    const bool whole32 = g.K % 32 == 0 && (g.ktotal == 0 || g.ktotal % 32 == 0);
-    return (a_plain && whole32 && g.K >= 2048) ? 2 * kSlot : kSlot;
+    return (a_plain && g.K % (2 * kSlot) == 0 && g.K >= 2048) ? 2 * kSlot : kSlot;
 }
 
 // One block per tile.
@@ -238,10 +238,12 @@ constexpr int64_t kSplitFloatsPerCu = 65536;
 // and the least K that splits: a split costs its sum's launch, 2.3 us, and a
 // 64x128 tile alone on a CU takes 0.032 us per k.
 constexpr int64_t kMinFewDepth = 48, kMinFewK = 128;
-// Time of two 128x128 blocks sharing a CU against one 256x256 block on it,
-// from the FP32 MFMA tiles' rates; these run 0.106 us per k at 32 x 512^3,
-// its fixed part included, against 0.15 at 4096^3.  A ragged output takes the
-// large tile when its rounds of blocks, so weighted, are no more.
+// Time of a round of two 128x128 blocks per CU against one of a 256x256 block
+// each: 0.50 to 0.57 for ragged single products and batches of K from 200 to
+// 2200 (4095x300x4095 0.51, 700x600x700 x 24 0.55, 3318x2176x6109 0.53), 0.44
+// at the least.  A ragged output takes the large tile when its rounds of
+// blocks, so weighted, are no more: one round against two (5000x1000x3000 161 us,
+// 177 on 128x128), not two against three (5348x192x4570 78, 67).
 constexpr double kSmallPairOverLarge = 0.575;
 
 // Which kernel a product runs.  Tile choice:
@@ -256,18 +258,21 @@ constexpr double kSmallPairOverLarge = 0.575;
 //     K-slices, when S*tiles reaches half the CUs or at least the block
 //     count of the tile it replaces;
 //   - else 64x128 when 128x128 would give fewer than two blocks per CU and
-//     64x128 divides the shape (a CU with one block then has two), else
-//     128x128;
+//     64x128 divides the shape, whole pairs of slots in K (a CU with one block
+//     then has two), else 128x128.  Other K would run as well on it: as it is
+//     and on 64x128, us, 1024x1000x1024 29.0 and 26.8, 1024x500x2048 31.1 and
+//     26.7, 1920x700x1280 33.9 and 35.6, but batches lose (448x700x896 x 9 39.7
+//     and 46.8, 1024x300x1024 x 3 17.7 and 19.6);
 //   - but 64x128 at any shape of 64 rows or more that leaves most CUs without
 //     a block: half a 128x128 block's work on twice the CUs.  A single matrix
 //     of at most a tile per four CUs (beyond, 128x128 in slices is as fast:
-//     700^3 17.5 us, 18.7 on 64x128), split for at most one block per CU in
+//     700^3 16.9 us, 16.8 on 64x128), split for at most one block per CU in
 //     slices of at least kMinFewDepth; a K below kMinFewK and a batch, which do
 //     not split, while their tiles have a CU each.  128x128 / 64x128, us:
-//     64^3 6.8 / 6.1, 200x400x300 12.2 / 9.1, 300x784x500 13.8 / 11.9,
-//     300x500x100 13.2 / 9.2, 96x6144x96 22.1 / 18.8, 1000x64x1000 7.8 / 7.1,
-//     batches 32 of 100x128x100 9.9 / 8.4, 16 of 300^3 18.3 / 15.2, 8 of
-//     200x200x700 13.9 / 12.0;
+//     64^3 6.9 / 6.3, 200x400x300 12.1 / 9.3, 300x784x500 13.7 / 12.4,
+//     300x500x100 13.0 / 9.3, 96x6144x96 22.0 / 18.7, 1000x64x1000 8.0 / 7.3,
+//     batches 32 of 100x128x100 10.0 / 8.8, 16 of 300^3 16.9 / 15.3, 8 of
+//     200x200x700 13.1 / 11.7;
 //   - a single matrix whose tile gives at most one block per CU splits K
 //     over that tile (above);
 //   - then stream-K on the 256x256 tile (below) replaces the plan where it
@@ -403,15 +408,19 @@ GemmPlan plan_gemm_tiles(const GemmArgs &g, bool a_plain, bool a_trans, bool b_p
 // fewer tiles than CUs that no power-of-two K split fills (3072^3: 144).
 //
 // The choice compares estimated times in k steps of one 256x256 tile on one
-// CU (0.15 us at 4096^3): the plan above by its rounds of
+// CU (0.16 us at 4096^3): the plan above by its rounds of
 // blocks, and stream-K by its even share plus kStreamKCost for the pieces'
 // extra traffic (two 256 KiB pieces per split tile written, read back and
 // added, at most one split tile per block), the fix-up launch and a block's
 // extra segment starts.  The 128x128 and 64x128 tiles cost 0.30 and 0.175
-// of a large k step per k (their rates and areas; alone on a CU a 64x128 block
-// takes 0.032 us per k, 0.21 of one).  Against every tile and split of 30
-// shapes the choice is the fastest or within a few percent, at most 12% off
-// (512x4096x4096 113 us, 101 in 8 large slices; 2048^3 109 and 101).  Stream-K needs
+// of a large k step per k (their rates and areas; alone on a CU 2048^3 takes
+// 0.048 us per k on 128x128, a 64x128 block 0.029).  Against every tile and up
+// to 16 slices of 388 products of random shape, layout and batch the plan is
+// the fastest for half, within 15% for nine in ten and 3.5% off in the mean;
+// the worst split a short K that 128x128 tiles already give a round
+// (5133x256x622 32.7 us in 2 slices, 17.3 whole; 5950x387x214 25.5 in 3, 16.0
+// on 64x128 whole); of the large ones 512x4096x4096 115 us, 104 in 2 slices of
+// 128x128, and 2048^3 114 on stream-K, 98.5 on 128x128 whole.  Stream-K needs
 // tiles at least 85% covered, no K split of its own (ktotal), and at least
 // kStreamKMinWork k steps per CU.
 constexpr double kStreamKCost = 150.0;

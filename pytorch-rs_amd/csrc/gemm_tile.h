@@ -19,7 +19,7 @@
 // back a rounding a slot, which operands with many zeros (a relu's output
 // under dropout, one-hot rows) show: with a 0.02 share of nonzeros it is
 // behind fp32 MFMA (1.1 times its error), and with the small products added
-// straight to `acc` in half the slots, which was faster (583 us at 4096^3),
+// straight to `acc` in half the slots, which was faster (580-630 us at 4096^3),
 // from a share of 0.35 down (1.6 times at 0.02).  The price is registers: a
 // 256x256 tile has room for one sum only, so it is computed as two halves of
 // 256x128, each splitting A again.
@@ -35,8 +35,9 @@
 // The one case behind is an output, or a K slice's part of it, that is a single
 // nonzero product: the three products left out, below 2^-24 of it together,
 // take a diagonal operand from 2.52e-8 to 2.59e-8 (4% of such outputs are the
-// neighbour of the correctly rounded product; K = 1 goes to fp32 MFMA) and [64, 512] @ [512, 200] in 8
-// slices with a 0.02 share of nonzeros from 5.52e-8 to 5.58e-8.
+// neighbour of the correctly rounded product; K = 1 goes to fp32 MFMA) and
+// [64, 512] @ [512, 200] in 8 slices with a 0.02 share of nonzeros from 5.52e-8
+// to 5.58e-8.
 //
 // An output of a tile depends on its row of A and its column of B alone,
 // wherever they stand in it.  The order of the products is not symmetric in A
@@ -54,9 +55,10 @@
 // (950 on the fp32 MFMA build; 1,630 where every such tile was computed
 // again), all values that small: 1,110-1,140 (950; 1,590).
 //
-// What bounds it: the card's power.  At 4096^3 random values run 640-670 us
-// (1,230-1,290 TFLOP/s of bf16), zeros in far less at a higher clock.  The fp32
-// MFMA kernel this replaced took 950 us.
+// What bounds it: the card's power.  At 4096^3 random values run 615-700 us by
+// layout and card (1,180-1,340 TFLOP/s of bf16; 580-630 with one sum in a 256x256
+// tile), where the MFMAs alone would take 466.  The fp32 MFMA kernel this
+// replaced took 935-970 us.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -309,8 +311,10 @@ struct SlotOperand {
 };
 
 // A BM x BN tile of C on WGM x WGN waves, each (BM/WGM) x (BN/WGN) as 32x32
-// MFMA tiles.  AHEAD slots are on their way from memory in registers (the
-// depth is not what bounds it: 1, 2 and 3 measured within 1%).  AKC, BKC: the operand is contiguous along k.
+// MFMA tiles, and PARTS of them side by side, one after the other.  AHEAD slots
+// are on their way from memory in registers (the depth is not what bounds it:
+// 4096^3 by layout 667, 673 and 632 us with 1, 679, 660 and 663 with 2).  AKC,
+// BKC: the operand is contiguous along k.
 template <int BM, int BN, int WGM, int WGN, int AHEAD, bool AKC, bool BKC, int PARTS = 1>
 struct GemmTile {
     static constexpr int NT = WGM * WGN * 64, WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
@@ -376,7 +380,7 @@ struct GemmTile {
     // anyway, and not behind the last whole slot.
     //
     // Slot t is computed from one of three LDS buffers while slot t + 2 is split from
-    // registers into another and slot t + 3 is loaded into those
+    // registers into another and slot t + 2 + AHEAD is loaded into those
     // registers.  Slot t + 1's buffer was complete at the barrier before, so the
     // fragments a slot starts with are read before the barrier that ends the
     // slot ahead of it.  A wave walks its rows of MFMA tiles; the reads for
