@@ -374,7 +374,7 @@ def matmul_only(args) -> int:
     from trs_backend import abi
     from trs_backend.abi import DeviceArray, check, layout_of
     from trs_backend.configs import generate
-    from trs_backend.timing import time_region
+    from trs_backend.timing import product_rates, time_region
 
     K = 4096
     dA, dB = DeviceArray.from_numpy(generate("matmul", "A")), DeviceArray.from_numpy(generate("matmul", "B"))
@@ -387,8 +387,8 @@ def matmul_only(args) -> int:
     ms = time_region(mm, reps=args.steps, warmup=args.warmup)
     tf = 2 * K ** 3 / (ms * 1e-3) / 1e12
     log(f"matmul 4096^3: {ms:.3f} ms avg over {args.steps} launches -> {tf:.1f} TFLOPS")
-    print(json.dumps({"workload": "matmul_4096", "flop_per_launch": 2 * K ** 3, "ms_avg": ms, "TFLOPS": tf,
-                      "frac_mfma_peak": tf / FP32_MFMA_PEAK_TFLOPS}), flush=True)
+    print(json.dumps({"workload": "matmul_4096", "flop_per_launch": 2 * K ** 3, "ms_avg": ms, **product_rates(tf)}),
+          flush=True)
     return 0
 
 

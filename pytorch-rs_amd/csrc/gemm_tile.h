@@ -336,15 +336,15 @@ struct GemmTile {
     gt_lds lds;
     int64_t lda, ldb;
     int64_t astep, bstep;
-    int lane, wm0, wn0;
+    int lane, wave, wm0, wn0;
 
     __device__ __forceinline__ explicit GemmTile(gt_lds l) : lds(l) {}
 
     // What the waves of a block tell one another: each posts a word (the same in
     // all its lanes) ahead of a barrier, and reads the or of them behind it.  All
     // post every time, so nothing has to be cleared.
-    __device__ __forceinline__ void post(Notice n, uint32_t word, unsigned tid) const {
-        ((gt_lds_words)(lds + kNotices))[n * NW + (tid >> 6)] = word;
+    __device__ __forceinline__ void post(Notice n, uint32_t word) const {
+        ((gt_lds_words)(lds + kNotices))[n * NW + wave] = word;
     }
     __device__ __forceinline__ uint32_t posted(Notice n) const {
         uint32_t any = 0;
@@ -456,7 +456,7 @@ struct GemmTile {
         };
         // The first slots are in LDS: the first fragments, and whether to give up.
         const auto first = [&](int slots, const Slot &s0, const Slot &s1) {
-            post(kFirstLost, in_wave((lost & 0xffffu) != 0), tid);
+            post(kFirstLost, in_wave((lost & 0xffffu) != 0));
             __syncthreads();
             read_a(0, 0, A[0]);
 #pragma unroll
@@ -596,7 +596,7 @@ struct GemmTile {
         const gt_lds_floats most = (gt_lds_floats)(lds + kSurvey), tiny = most + BM + BN;
         bool none = false;
         for (int i = tid; i < BM + BN; i += NT) none |= tiny[i] != 0.f && most[i] < kLeast;
-        post(kFails, in_wave(none), tid);
+        post(kFails, in_wave(none));
         __syncthreads();
         return posted(kFails);
     }
@@ -662,7 +662,7 @@ struct GemmTile {
                                              int64_t k1, float *ws, unsigned tid) {
         lda = args.lda, ldb = args.ldb;
         lane = tid & 63;
-        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         wm0 = (wave / WGN) * WM;
         wn0 = (wave % WGN) * WN;
         const int64_t Kb = args.ktotal ? imin(args.K, args.ktotal - batch * args.K) : args.K;
@@ -686,9 +686,10 @@ struct GemmTile {
             uint32_t lost;
             fp32 = split_slots(whole, tail, tid, lost);
             // What follows works its lane values out again, so that the slot loop
-            // does not keep them live.
-            asm volatile("" : "+v"(tid));
-            lane = tid & 63;
+            // does not keep them live (nor the lane's number itself).
+            lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+            asm volatile("" : "+v"(lane));
+            tid = (unsigned)(wave * 64 + lane);
             if (__builtin_expect(!fp32, 1)) {
                 // A non-finite accumulator leaves a non-finite sum of them.
                 float sum[4] = {0.f, 0.f, 0.f, 0.f};
@@ -703,7 +704,7 @@ struct GemmTile {
                         }
                 const float s = (sum[0] + sum[1]) + (sum[2] + sum[3]);
                 const bool bad = !(__builtin_fabsf(s) < __builtin_inff());
-                post(kResult, in_wave((lost & 0xffffu) != 0) | in_wave(bad) << 1, tid);
+                post(kResult, in_wave((lost & 0xffffu) != 0) | in_wave(bad) << 1);
                 __syncthreads();
                 const uint32_t result = posted(kResult);
                 fp32 = result & 2;
@@ -712,7 +713,7 @@ struct GemmTile {
                     int slots = whole, rest = tail;  // nothing of this ahead of the slot loop
                     asm volatile("" : "+s"(slots), "+s"(rest));
                     survey(slots, rest, tid);
-                    post(kFails, in_wave(harmed(slots, rest)), tid);
+                    post(kFails, in_wave(harmed(slots, rest)));
                     __syncthreads();
                     fp32 = posted(kFails);
                 }

@@ -20,10 +20,9 @@ import numpy as np
 from . import abi
 from .abi import DeviceArray, check, layout_of
 from .configs import generate
-from .timing import time_launches, time_region
+from .timing import product_rates, time_launches, time_region
 
 HBM_PEAK_GBS = 8000.0
-FP32_MFMA_PEAK_TFLOPS = 157.3
 
 
 def _spread(times_ms: list[float], scale: float = 1e3, unit: str = "us") -> dict:
@@ -219,8 +218,8 @@ def matmul(log, reps: int = 20) -> dict:
     med = time_region(mm, reps, warmup=int(GEMM_WARMUP_MS / 1.0))
     t = time_launches(mm, reps)
     tf = 2 * K ** 3 / (med * 1e-3) / 1e12
-    out["matmul_4096"] = {"ms_avg": med, "ms_min_single_launch": min(t), "TFLOPS": tf,
-                          "frac_mfma_peak": tf / FP32_MFMA_PEAK_TFLOPS, "spread": _spread(t, 1.0, "ms"),
+    out["matmul_4096"] = {"ms_avg": med, "ms_min_single_launch": min(t), **product_rates(tf),
+                          "spread": _spread(t, 1.0, "ms"),
                           "output_checksum": _checksum(dC, K * K)}
     log(f"matmul 4096^3: {med:.3f} ms, {tf:.1f} TFLOPS")
     Ab, Bb = generate("matmul", "Ab"), generate("matmul", "Bb")
@@ -234,8 +233,8 @@ def matmul(log, reps: int = 20) -> dict:
     med = time_region(bmm, reps * 3, warmup=int(GEMM_WARMUP_MS / 0.08))
     t = time_launches(bmm, reps * 3)
     tf = 2 * 32 * 512 ** 3 / (med * 1e-3) / 1e12
-    out["matmul_batched_32x512"] = {"ms_avg": med, "ms_min_single_launch": min(t), "TFLOPS": tf,
-                                    "frac_mfma_peak": tf / FP32_MFMA_PEAK_TFLOPS, "spread": _spread(t, 1.0, "ms"),
+    out["matmul_batched_32x512"] = {"ms_avg": med, "ms_min_single_launch": min(t), **product_rates(tf),
+                                    "spread": _spread(t, 1.0, "ms"),
                                     "output_checksum": _checksum(dCb, 32 * 512 * 512)}
     log(f"batched matmul 32x512^3: {med:.3f} ms, {tf:.1f} TFLOPS")
     return out
@@ -308,8 +307,8 @@ def matmul_shapes(log, reps: int = 100) -> dict:
             rate = f"{gbs:.0f} GB/s ({gbs / HBM_PEAK_GBS:.2f})"
         else:
             tf = 2 * M * N * K / (us * 1e-6) / 1e12
-            entry.update({"TFLOPS": tf, "frac_mfma_peak": tf / FP32_MFMA_PEAK_TFLOPS})
-            rate = f"{tf:.1f} TFLOPS ({tf / FP32_MFMA_PEAK_TFLOPS:.2f})"
+            entry.update(product_rates(tf))
+            rate = f"{tf:.1f} TFLOPS ({entry['frac_bf16_mfma_peak']:.2f} of bf16 MFMA)"
         out[name] = entry
         log(f"matmul {name}: {us:.1f} us, {rate}, tile {tm.value}x{tn.value}x{tk.value} splits {sp.value}")
         del sets

@@ -15,10 +15,9 @@ from __future__ import annotations
 import numpy as np
 
 from .configs import generate
-from .timing import time_launches, time_region
+from .timing import product_rates, time_launches, time_region
 
 GEMM_FLOP = 2 * (3 * 8192 * 4096 * 4096 + 3 * 8192 * 4096 * 1024)
-FP32_MFMA_PEAK_TFLOPS = 157.3
 
 
 def build(device: str = "cuda", fused: bool = True):
@@ -77,7 +76,7 @@ def run(log, reps: int = 20) -> dict:
     same = _bits(lf) == _bits(le) and all(_bits(a.grad) == _bits(b.grad) for a, b in ((x, xe), (w1, w1e), (w2, w2e)))
     log(f"mlp eager activation: {med_eager:.3f} ms/step; fused and eager loss and gradients bit-identical: {same}")
     return {"ms_avg": med, "ms_min_single_step": t[0], "ms_median_single_step": t[len(t) // 2],
-            "ms_max_single_step": t[-1], "gemm_flop_per_step": GEMM_FLOP, "TFLOPS": tf,
-            "frac_mfma_peak": tf / FP32_MFMA_PEAK_TFLOPS, "loss": loss, "grad_checksums": grad_sums,
+            "ms_max_single_step": t[-1], "gemm_flop_per_step": GEMM_FLOP, **product_rates(tf),
+            "loss": loss, "grad_checksums": grad_sums,
             "activation": "fused (bias add, relu, dropout-apply: one FusedBackward0 node)",
             "eager_activation_ms_avg": med_eager, "fused_equals_eager_bitwise": same}

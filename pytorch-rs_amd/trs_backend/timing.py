@@ -6,6 +6,17 @@ from ctypes import POINTER, c_float, c_int, c_void_p
 
 from .abi import check, lib
 
+FP32_MFMA_PEAK_TFLOPS = 157.3
+BF16_MFMA_PEAK_TFLOPS = 2516.6  # dense: 16 times the former
+
+
+def product_rates(tflops: float) -> dict:
+    """The rate of fp32 products, as a share of the FP32 MFMA peak, which the
+    tiles pass, and as what runs: six bf16 products each, on the bf16 peak."""
+    return {"TFLOPS": tflops, "frac_mfma_peak": tflops / FP32_MFMA_PEAK_TFLOPS, "bf16_TFLOPS": 6 * tflops,
+            "frac_bf16_mfma_peak": 6 * tflops / BF16_MFMA_PEAK_TFLOPS}
+
+
 _hip = ctypes.CDLL("libamdhip64.so.7")
 _hip.hipEventCreate.argtypes = [POINTER(c_void_p)]
 _hip.hipEventCreate.restype = c_int
