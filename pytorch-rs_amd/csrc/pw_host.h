@@ -445,31 +445,6 @@ inline int plan_pointwise(const trs_layout *lo, float *out, int nin, const void 
                     else if (is[i][tdim] == 0) plan->once |= 1u << i;
                 }
             }
-            // Through LDS where the output's rows are not whole lines apart, the
-            // one transposed operand and every other are floats, and the 64 x
-            // 256 tiles are at least kLdsCover full.  Fused (a + b) * c.mT,
-            // through LDS against the direct tiles, in us: [60, 500, 1001] 62 /
-            // 119, [20, 1023, 999] 49 / 78, [16, 64, 300] (0.59 full) 7.0 /
-            // 10.6; emptier tiles lose: [33, 77, 901] (0.53) 11.4 / 8.8, [10,
-            // 300, 130] (0.24) 9.3 / 5.5.
-            bool whole_lines = true, floats = true;
-            for (int d = 0; d < inner; d++) whole_lines &= os[d] % 32 == 0;
-            for (int i = 0; i < nin; i++) floats &= elem_bytes[i] == 4;
-            const auto cover = [](int64_t n, int64_t tile) { return (double)n / (double)((n + tile - 1) / tile * tile); };
-            if (vec && nt == 1 && floats && !whole_lines && size[tdim] >= 4 && size[inner] >= 4 &&
-                cover(size[tdim], kLdsT) * cover(size[inner], kLdsX) >= kLdsCover) {
-                plan->lds = true;
-                plan->held = plan->once = plan->xbc = 0;
-                g.groups = g.rows;
-                g.ttiles = (size[tdim] + kLdsT - 1) / kLdsT;
-                g.chunks = g.ttiles * ((size[inner] + kLdsX - 1) / kLdsX);
-                const bool small = g.groups * g.chunks <= (int64_t)UINT32_MAX;
-                g.fdchunks = make_fast_div(small ? (uint32_t)g.chunks : 1u);
-                g.fdttiles = make_fast_div(small ? (uint32_t)g.ttiles : 1u);
-                plan->block = 64 * kLdsWaves;
-                plan->grid = std::min<int64_t>(g.groups * g.chunks, want);
-                return TRS_OK;
-            }
             // When an operand is held, each block walks the largest of 8, 4
             // or 2 tuples that divides the tuple count (the held operand is
             // then loaded once for all of them); else one tuple per block.
@@ -480,6 +455,45 @@ inline int plan_pointwise(const trs_layout *lo, float *out, int nin, const void 
                         plan->walk = w;
                         break;
                     }
+            // Through LDS where the output's rows are not whole lines apart, the
+            // one transposed operand and every other are floats, the 64 x 256
+            // tiles are at least kLdsCover full, and they give every CU a block
+            // (5 of 8 where a second operand is read whole, which gives a block
+            // more to move): a block of the direct tiles is done sooner, and there
+            // are more of them, except where they walk 4 or 8 tuples and are few.
+            // Direct / through LDS, in us, fused (a + b) * c.mT:
+            //   many blocks   [60, 500, 1001] 118 / 62, [58, 668, 805] 123 / 67,
+            //                 [22, 256, 748] (264) 15.3 / 11.2
+            //   fewer         [9, 448, 703] (189) 10.2 / 13.0, [5, 896, 207] (70)
+            //                 5.2 / 10.8, [13, 64, 421] (26) 4.5 / 8.3
+            //   a walk of 8   [8, 709, 420] (192) 22.4 / 8.6, [8, 128, 876] (64)
+            //                 14.4 / 7.0, [32, 112, 324] (128) 15.5 / 7.4
+            //   less full     [58, 528, 111] (0.40) 15.2 / 20.6, [55, 596, 78] (0.28)
+            //                 11.7 / 18.1, [61, 263, 102] (0.33) 8.2 / 11.9
+            // and y + c.mT: [38, 192, 433] (228) 16.0 / 11.4, [43, 64, 933] (172)
+            // 12.1 / 9.1, [2, 960, 802] (120) 7.1 / 9.3, [8, 448, 385] (112) 7.2 / 8.2.
+            bool whole_lines = true, floats = true;
+            for (int d = 0; d < inner; d++) whole_lines &= os[d] % 32 == 0;
+            for (int i = 0; i < nin; i++) floats &= elem_bytes[i] == 4;
+            const auto tiles_of = [](int64_t n, int64_t tile) { return (n + tile - 1) / tile; };
+            const int64_t lds_t = tiles_of(size[tdim], kLdsT), lds_tuple = lds_t * tiles_of(size[inner], kLdsX);
+            const double cover = (double)(size[tdim] * size[inner]) / (double)(lds_tuple * kLdsT * kLdsX);
+            const int64_t lds_least = __builtin_popcount(g.streamed) > 1 ? (int64_t)cu_count * 5 / 8 : cu_count;
+            if (vec && nt == 1 && floats && !whole_lines && size[tdim] >= 4 && size[inner] >= 4 && cover >= kLdsCover &&
+                (g.rows * lds_tuple >= lds_least || plan->walk >= 4)) {
+                plan->lds = true;
+                plan->held = plan->once = plan->xbc = 0;
+                plan->walk = 1;
+                g.groups = g.rows;
+                g.ttiles = lds_t;
+                g.chunks = lds_tuple;
+                const bool small = g.groups * g.chunks <= (int64_t)UINT32_MAX;
+                g.fdchunks = make_fast_div(small ? (uint32_t)g.chunks : 1u);
+                g.fdttiles = make_fast_div(small ? (uint32_t)g.ttiles : 1u);
+                plan->block = 64 * kLdsWaves;
+                plan->grid = std::min<int64_t>(g.groups * g.chunks, want);
+                return TRS_OK;
+            }
             g.groups = g.rows / plan->walk;
             g.ttiles = (size[tdim] + kXposeBT - 1) / kXposeBT;
             const int64_t xtiles = (size[inner] + kXposeBX - 1) / kXposeBX;

@@ -95,30 +95,62 @@ def test_transposed_operand_at_every_edge(nb, t, x):
     _same(torch_rs.fuse(lambda p, q: p * q)(torch_rs.tensor(col, device="cuda"), dc.mT).numpy(), col * ct)
 
 
-# Those that run on the tiles through LDS (64 t by 256 x, at least 0.55 full):
-# t and x around the tiles' edges, a last tile of one row or column, every
-# residue mod 4, and the least full.
-THROUGH_LDS = [(2, 130, 1001), (2, 36, 253), (1, 64, 144), (1, 64, 145), (3, 63, 146), (1, 63, 147), (1, 62, 255),
-               (2, 64, 254), (1, 129, 1023), (1, 130, 1021), (2, 131, 1022), (1, 64, 769), (1, 64, 770), (1, 64, 771),
-               (1, 127, 511), (2, 125, 700), (3, 128, 510)]
+# Those that run on the tiles through LDS (64 t by 256 x, at least 0.55 full, and a
+# batch of 4 or 8, which the direct tiles would walk): t and x around the tiles'
+# edges, a last tile of one row or column, every residue mod 4, and the least full.
+THROUGH_LDS = [(8, 36, 253), (4, 64, 144), (4, 64, 145), (4, 63, 146), (4, 63, 147), (4, 62, 255), (4, 64, 254),
+               (4, 129, 1023), (4, 130, 1021), (8, 131, 1022), (4, 64, 769), (4, 64, 770), (4, 64, 771), (4, 127, 511),
+               (4, 125, 700), (8, 128, 510), (4, 130, 1001)]
+
+
+def _lds_operands(nb, t, x):
+    rng = np.random.default_rng(nb + 3 * t + 7 * x)
+    return _normal(rng, nb, 1, x), _normal(rng, 1, t, x), _normal(rng, nb, x, t), _normal(rng, nb, t, 1), _normal(rng, 1)
+
+
+def _runs_through_lds(nb, t, x, roles=True):
+    """(a + b) * c.mT fused, or c.mT and a whole operand eager."""
+    whole, ct = layout_of((nb, t, x)), layout_of((nb, t, x), (t * x, 1, t))
+    lays = [layout_of((nb, 1, x)), layout_of((1, t, x)), ct] if roles else [whole, ct]
+    return abi.pointwise_plan_access(lays, whole, roles=roles) == (True, True)
 
 
 @pytest.mark.parametrize("nb,t,x", THROUGH_LDS)
 def test_lds_tiles_at_every_edge(nb, t, x):
     import torch_rs
-    lays = [layout_of((nb, 1, x)), layout_of((1, t, x)), layout_of((nb, t, x), (t * x, 1, t))]
-    assert abi.pointwise_plan_access(lays, layout_of((nb, t, x)), roles=True) == (True, True)
-    rng = np.random.default_rng(nb + 3 * t + 7 * x)
-    a, b, c = _normal(rng, nb, 1, x), _normal(rng, 1, t, x), _normal(rng, nb, x, t)
-    da, db, dc = (torch_rs.tensor(v, device="cuda") for v in (a, b, c))
+    assert _runs_through_lds(nb, t, x)
+    host = a, b, c, col, scalar = _lds_operands(nb, t, x)
+    da, db, dc, dcol, ds = (torch_rs.tensor(v, device="cuda") for v in host)
     ct, full = c.transpose(0, 2, 1), a + b
     _same(torch_rs.fuse(lambda p, q, r: (p + q) * r)(da, db, dc.mT).numpy(), full * ct)
-    _same((torch_rs.tensor(full, device="cuda") + dc.mT).numpy(), full + ct)
-    col, scalar = _normal(rng, nb, t, 1), _normal(rng, 1)
-    dcol, ds = torch_rs.tensor(col, device="cuda"), torch_rs.tensor(scalar, device="cuda")
     # five inputs: the others are read after the barrier
     five = torch_rs.fuse(lambda p, q, r, u, v: ((p + q) * r - u) * v)
     _same(five(da, db, dc.mT, dcol, ds).numpy(), (full * ct - col) * scalar)
+
+
+@pytest.mark.parametrize("nb,t,x", [(128, 61, 413), (256, 64, 255), (65, 80, 1021), (43, 130, 511), (257, 36, 254)])
+def test_lds_tiles_eager(nb, t, x):
+    """From a block per CU (256) on, whatever the batch."""
+    import torch_rs
+    assert _runs_through_lds(nb, t, x, roles=False)
+    a, b, c, _, _ = _lds_operands(nb, t, x)
+    full, ct = a + b, c.transpose(0, 2, 1)
+    got = torch_rs.tensor(full, device="cuda") + torch_rs.tensor(c, device="cuda").mT
+    _same(got.numpy(), full + ct)
+
+
+def test_loop_over_lds_tiles_of_a_walked_batch():
+    """Fewer blocks than tiles: each block takes several LDS tiles."""
+    import torch_rs
+    nb, t, x = 4, 150, 601
+    assert _runs_through_lds(nb, t, x)
+    a, b, c, _, _ = _lds_operands(nb, t, x)
+    da, db, dc = (torch_rs.tensor(v, device="cuda") for v in (a, b, c))
+    check(abi.lib.trs_debug_pointwise_grid_cap(3))
+    try:
+        _same(torch_rs.fuse(lambda p, q, r: (p + q) * r)(da, db, dc.mT).numpy(), (a + b) * c.transpose(0, 2, 1))
+    finally:
+        check(abi.lib.trs_debug_pointwise_grid_cap(0))
 
 
 def test_transposed_views_at_any_float_and_higher_rank():

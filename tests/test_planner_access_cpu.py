@@ -34,11 +34,28 @@ def test_byte_operands_are_vectors_on_whole_quads(cols):
 def test_transposed_operands_vector_and_lds(nb, t, x):
     a, b, c = layout_of((nb, 1, x)), layout_of((1, t, x)), layout_of((nb, t, x), (t * x, 1, t))
     out = layout_of((nb, t, x))
-    plan = abi.pointwise_plan([a, b, c], out, roles=True)
-    assert plan.variant == XPOSE_VARIANT
-    # rows off the 128-byte lines and 64 x 256 tiles (t by x) at least 0.55 full
-    lds = (nb, t, x) in THROUGH_LDS
-    for roles in (False, True):
-        assert access(a, b, c, out=out, roles=roles) == (True, lds)
+    assert abi.pointwise_plan([a, b, c], out, roles=True).variant == XPOSE_VARIANT
+    assert access(a, b, c, out=out, roles=True) == (True, (nb, t, x) in THROUGH_LDS)
+    # without roles nothing is walked, and these are few blocks
+    assert access(a, b, c, out=out) == (True, False)
     # two transposed operands stay in registers
     assert access(c, c, b, out=out, roles=True) == (True, False)
+
+
+# 64 x 256 tiles (t by x): from a block per CU on, or where the direct tiles would
+# walk 4 or 8 tuples of a batch; 0.55 full or more, and rows off the 128-byte lines.
+@pytest.mark.parametrize("nb,t,x,lds", [(255, 64, 250, False), (256, 64, 250, True), (255, 64, 256, False),
+                                        (9, 448, 703, False), (12, 448, 703, True), (22, 256, 748, True),
+                                        (58, 528, 111, False), (512, 64, 140, False), (512, 64, 141, True),
+                                        (6, 709, 420, False), (10, 709, 420, False), (8, 709, 420, True)])
+def test_when_a_transposed_operand_goes_through_lds(nb, t, x, lds):
+    a, b, c = layout_of((nb, 1, x)), layout_of((1, t, x)), layout_of((nb, t, x), (t * x, 1, t))
+    assert access(a, b, c, out=layout_of((nb, t, x)), roles=True) == (True, lds)
+
+
+@pytest.mark.parametrize("nb,t,x,lds", [(159, 64, 250, False), (160, 64, 250, True), (8, 448, 385, False),
+                                        (43, 64, 933, True), (1, 1000, 777, False), (1, 3000, 3001, True)])
+@pytest.mark.parametrize("roles", [False, True])
+def test_with_a_second_whole_operand_through_lds_from_fewer_blocks(nb, t, x, lds, roles):
+    y, c = layout_of((nb, t, x)), layout_of((nb, t, x), (t * x, 1, t))
+    assert access(y, c, out=y, roles=roles) == (True, lds)
