@@ -134,6 +134,19 @@ inline int rows_lanes(uint32_t streamed, int nin, const int *elem_bytes, int nou
     return kRowLanesMax;
 }
 
+// Whether a vector rows kernel whose rows start off 16 bytes takes its widest
+// blocks: every block's piece of a row then begins and ends inside a 128-byte
+// line that another block, on another XCD, writes the rest of, so few and long
+// pieces, where the row fills them.  Measured, in us, 64 lanes / 256: the copy of
+// [8192, 998] out of [8192, 1001] 14.5 / 12.8 (13.2 with scalar accesses), x + row
+// over [2539, 7843] 31.0 / 28.6, [512, 65537] 52.1 / 45.8, [8191, 8190] 96.5 /
+// 89.4, [6912, 3679] (0.90 full) 39.8 / 37.3; half empty blocks lose: [20000, 515]
+// 18.6 / 19.8, [60000, 131] 18.6 / 37.5.
+inline bool ragged_rows_wide(int64_t cols) {
+    const int64_t chunk = 4 * kRowLanesMax;
+    return (double)cols >= 0.85 * (double)((cols + chunk - 1) / chunk * chunk);
+}
+
 // `elem_bytes[i]` is 4 for f32 inputs and 1 for u8 inputs.  A program with
 // several outputs passes outputs 1.. in `more` (nout - 1 of them); they share
 // the output layout `lo`.  `roles`: the launcher can run pw_xpose specialised
@@ -388,6 +401,7 @@ inline int plan_pointwise(const trs_layout *lo, float *out, int nin, const void 
             plan->vec = vec && size[inner] >= 4;
             plan->aligned &= size[inner] % 4 == 0;
             plan->block = plan->vec ? rows_lanes(g.streamed, nin, elem_bytes, nout) : 256;
+            if (plan->vec && !plan->aligned && ragged_rows_wide(size[inner])) plan->block = kRowLanesMax;
             g.chunkcols = plan->vec ? 4 * plan->block : 0;
             g.rows = numel / size[inner];
             const int64_t chunk = plan->vec ? g.chunkcols : kRowChunk;

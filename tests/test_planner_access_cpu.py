@@ -59,3 +59,14 @@ def test_when_a_transposed_operand_goes_through_lds(nb, t, x, lds):
 def test_with_a_second_whole_operand_through_lds_from_fewer_blocks(nb, t, x, lds, roles):
     y, c = layout_of((nb, t, x)), layout_of((nb, t, x), (t * x, 1, t))
     assert access(y, c, out=y, roles=roles) == (True, lds)
+
+
+@pytest.mark.parametrize("cols,lanes", [(7843, 256), (1001, 256), (998, 256), (871, 256), (870, 64), (515, 64), (511, 64),
+                                        (131, 64), (37, 64), (3679, 256), (1025, 64), (1400, 64)])
+def test_ragged_rows_take_the_widest_blocks_where_they_fill_them(cols, lanes):
+    """Rows off 16 bytes; aligned ones keep the block for the bytes it moves."""
+    x, b = layout_of((300, cols)), layout_of((cols,))
+    base = [0x20000000004, 0x30000000000]
+    assert abi.pointwise_plan([x, b], x, bases=base).block == lanes
+    aligned = layout_of((300, 4096))
+    assert abi.pointwise_plan([aligned, layout_of((4096,))], aligned).block == 64
