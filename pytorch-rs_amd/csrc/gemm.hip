@@ -12,7 +12,7 @@
 // Three tiles (GemmTile), each in the four operand layouts and at any M, N
 // and K (rows past the edge repeat the last one and are not stored):
 //   256x256  two 256x128 halves one after the other, 8 waves of 64x64, one
-//            block per CU (108 KB of LDS)
+//            block per CU (111 KB of LDS)
 //   128x128  4 waves of 64x64, two blocks per CU, or where blocks do not fill
 //            the CUs twice 8 of 32x64, one per CU
 //   64x128   4 waves of 32x64, two blocks per CU

@@ -53,7 +53,8 @@
 // Lost bits in the first slots of rows that hold nothing larger go to fp32 MFMA
 // at once (useless()).  4096^3, one value of 2^-119 in every 64 rows: 905-935 us
 // (950 on the fp32 MFMA build; 1,630 where every such tile was computed
-// again), all values that small: 1,110-1,140 (950; 1,590).
+// again), all values that small: 1,110-1,140 (950; 1,590), a NaN in every 64 rows,
+// whose tiles are all computed twice, 1,700 (950).
 //
 // What bounds it: the card's power.  At 4096^3 random values run 615-700 us by
 // layout and card (1,180-1,340 TFLOP/s of bf16; 580-630 with one sum in a 256x256
