@@ -404,8 +404,7 @@ struct GemmTile {
         };
         typedef const gt_bf8 __attribute__((address_space(3))) *Frag;
         const gt_lds fa = lds + wm0 * 32 + lane * 16, fb = lds + kABytes + wn0 * 32 + lane * 16;
-        // The products (piece of A, piece of B), the smaller first: in a tile
-        // that keeps the first five apart their sum is added before the sixth.
+        // The products (piece of A, piece of B): five for `low`, the sixth for `acc`.
         static constexpr int PA[6] = {2, 1, 1, 0, 0, 0}, PB[6] = {0, 0, 1, 1, 2, 0};
         int cur = 0, nxt = kBuf, wr = 2 * kBuf;  // this slot's buffer, the next one's, the one being written
         gt_bf8 A[2][3], B[TN][3];
@@ -417,12 +416,13 @@ struct GemmTile {
 #pragma unroll
             for (int p = 0; p < 3; p++) B[j][p] = *(Frag)(fb + buf + p * OB::kPlane + j * 1024);
         };
-        // MORE: more slots may follow.  D: the registers holding slot t + 2.
-        const auto slot = [&]<bool MORE, int D>() {
+        // LEFT: the slots that follow this one, 2 for two or more.  D: the registers
+        // holding slot t + 2.
+        const auto slot = [&]<int LEFT, int D>() {
 #pragma unroll
             for (int i = 0; i < TM; i++) {
                 if (i + 1 < TM) read_a(cur, i + 1, A[(i + 1) & 1]);
-                else if (MORE) read_a(nxt, 0, A[TM & 1]);
+                else if (LEFT > 0) read_a(nxt, 0, A[TM & 1]);
 #pragma unroll
                 for (int p = 0; p < 6; p++)
 #pragma unroll
@@ -430,11 +430,13 @@ struct GemmTile {
                         gt_f16 &d = p < 5 ? low[i][j] : acc[i][j];
                         d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[i & 1][PA[p]], B[j][PB[p]], d, 0, 0, 0);
                     }
-                if constexpr (MORE) {
+                if constexpr (LEFT > 0) {
                     if (i == TM - 1) {
 #pragma unroll
                         for (int j = 0; j < TN; j++) read_b(nxt, j);
                     }
+                }
+                if constexpr (LEFT > 1) {
                     if (i == 0) oa.store_split(in[D].a, lds + wr, lost);
                     if (i == (TM > 1 ? 1 : 0)) {
                         oa.load(in[D].a, lda);
@@ -447,11 +449,11 @@ struct GemmTile {
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if constexpr (MORE && TM % 2 == 1) {
+            if constexpr (LEFT > 0 && TM % 2 == 1) {
 #pragma unroll
                 for (int p = 0; p < 3; p++) A[0][p] = A[1][p];
             }
-            __syncthreads();
+            if constexpr (LEFT > 1) __syncthreads();
             const int c = cur;
             cur = nxt, nxt = wr, wr = c;
         };
@@ -491,7 +493,7 @@ struct GemmTile {
                 clear();
                 put(s0, 0);
                 if (__builtin_expect(first(1, s0, s0), 0)) return true;
-                slot.template operator()<false, 0>();
+                slot.template operator()<0, 0>();
                 return false;
             }
         } else {
@@ -509,14 +511,24 @@ struct GemmTile {
         put(s0, 0);
         put(s1, kBuf);
         if (__builtin_expect(first(2, s0, s1), 0)) return true;
-        // Slot t takes registers t % AHEAD.
+        // Slot t takes registers t % AHEAD.  The last two slots of a short K split
+        // and load nothing: a load past the end is waited for, a memory latency for
+        // every tile (64^3 6.3 us with it, 5.6 without; batched 32 x 256x32x256 6.6
+        // and 5.7).  The large tile, whose K is long or whose store is, does not
+        // tell them apart: its loop comes out 5% slower with them (4096^3 645 us,
+        // 683).
+        constexpr int kEnd = PARTS == 1 ? 2 : 0;
         int t = 0;
 #pragma unroll 1
-        for (; t + 2 <= T; t += 2) {
-            slot.template operator()<true, 0>();
-            slot.template operator()<true, 1 % AHEAD>();
+        for (; t + 2 + kEnd <= T; t += 2) {
+            slot.template operator()<2, 0>();
+            slot.template operator()<2, 1 % AHEAD>();
         }
-        if (t < T) slot.template operator()<true, 0>();
+        if (t + 1 + kEnd == T) slot.template operator()<2, 0>();
+        if constexpr (kEnd) {
+            if (T > 1) slot.template operator()<1, 0>();
+            slot.template operator()<0, 0>();
+        }
         return false;
     }
 
