@@ -18,10 +18,10 @@
 //   64x128   4 waves of 32x64, two blocks per CU
 // The 4-wave 128x128 tile reads a third less from LDS per product, which
 // counts where the whole chip runs it and power sets the clock (batched
-// 32x512^3 57.6 us against 61.6, 1000x2047x1500 52.6 against 58.7, on one
+// 32x512^3 53.9 us against 58.3, 1000x2047x1500 48.7 against 58.0, on one
 // card); the 8-wave one issues its slot in half the instructions per wave, which
-// counts where one block has a CU to itself (700^3 17.6 us against 19.6,
-// 2048x100x2048 12.6 against 13.1).
+// counts where one block has a CU to itself (700^3 16.8 us against 19.1,
+// 2048x100x2048 11.8 against 12.2).
 // Blocks are remapped so that consecutive tiles share an XCD (each XCD has
 // its own L2), and tiles are walked in groups of kGroupM tile rows.
 #include <hip/hip_runtime.h>
@@ -266,13 +266,13 @@ constexpr double kSmallPairOverLarge = 0.575;
 //   - but 64x128 at any shape of 64 rows or more that leaves most CUs without
 //     a block: half a 128x128 block's work on twice the CUs.  A single matrix
 //     of at most a tile per four CUs (beyond, 128x128 in slices is as fast:
-//     700^3 16.9 us, 16.8 on 64x128), split for at most one block per CU in
+//     700^3 16.5 us, 16.1 on 64x128), split for at most one block per CU in
 //     slices of at least kMinFewDepth; a K below kMinFewK and a batch, which do
 //     not split, while their tiles have a CU each.  128x128 / 64x128, us:
-//     64^3 6.9 / 6.3, 200x400x300 12.1 / 9.3, 300x784x500 13.7 / 12.4,
-//     300x500x100 13.0 / 9.3, 96x6144x96 22.0 / 18.7, 1000x64x1000 8.0 / 7.3,
-//     batches 32 of 100x128x100 10.0 / 8.8, 16 of 300^3 16.9 / 15.3, 8 of
-//     200x200x700 13.1 / 11.7;
+//     64^3 6.5 / 5.9, 200x400x300 11.8 / 8.8, 300x784x500 13.4 / 12.0,
+//     300x500x100 12.8 / 8.7, 96x6144x96 21.6 / 18.0, 1000x64x1000 7.5 / 6.8,
+//     batches 32 of 100x128x100 9.5 / 8.2, 16 of 300^3 16.6 / 14.1, 8 of
+//     200x200x700 12.8 / 11.1;
 //   - a single matrix whose tile gives at most one block per CU splits K
 //     over that tile (above);
 //   - then stream-K on the 256x256 tile (below) replaces the plan where it
